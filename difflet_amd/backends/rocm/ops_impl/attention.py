@@ -113,19 +113,43 @@ def _valid_prefix_bounds(b, h, s_q, count, device):
     return torch.zeros_like(bound_max), bound_max
 
 
+def _two_segments(q, k, v, k2, v2, scale, causal, count) -> bool:
+    """Whether the joint kernel takes this call (keys in two segments, never concatenated):
+    bf16 / fp16 at head_dim 128, a positive scale, no causal mask, matching segments. Anything
+    else is concatenated and runs, or is refused, as attention() does."""
+    ts = (q, k, v, k2, v2)
+    return (not causal and scale > 0 and q.dtype in (torch.bfloat16, torch.float16)
+            and all(t.dim() == 4 and t.dtype == q.dtype and t.device == q.device
+                    and t.shape[:2] == q.shape[:2] and t.shape[3] == 128 for t in ts)
+            and q.device.type == "cuda" and k.shape == v.shape and k2.shape == v2.shape
+            and k.shape[2] > 0 and k.shape[2] + k2.shape[2] < 1 << 24
+            and (count is None or (torch.is_tensor(count) and count.numel() == q.shape[0])))
+
+
+def _joint(q, k, v, k2, v2, scale, causal, count, offset):
+    """Attention of q to [k | k2], keys [0, count + offset) when a count is given."""
+    scale = 1.0 if scale is None else float(scale)
+    if _two_segments(q, k, v, k2, v2, scale, causal, count):
+        if count is not None:
+            count = count.to(device=q.device, dtype=torch.int32).reshape(-1)
+        return library.attention_joint(q, k, v, k2, v2, float(scale), count, offset)
+    k = torch.cat([k, k2], dim=2)
+    v = torch.cat([v, v2], dim=2)
+    bounds = {}
+    if count is not None:
+        b, h, s_q, _ = q.shape
+        count = offset + count.to(torch.int32)
+        bounds = dict(zip(("bound_min", "bound_max"), _valid_prefix_bounds(b, h, s_q, count, q.device)))
+    return attention(q, k, v, scale=scale, causal=causal, **bounds)
+
+
 def joint_ring_attention(q, image_k, image_v, text_k, text_v, *, scale: float,
                          causal: bool = False, text_valid_len=None):
     """cp = 1: full joint attention over the keys [image | text]; with ``text_valid_len`` the
     keys [0, S_img + count) attend (right-padded text)."""
     _require_cp1("joint_ring_attention")
-    k = torch.cat([image_k, text_k], dim=2)
-    v = torch.cat([image_v, text_v], dim=2)
-    bounds = {}
-    if text_valid_len is not None:
-        b, h, s_q, _ = q.shape
-        count = image_k.shape[2] + text_valid_len.to(torch.int32)
-        bounds = dict(zip(("bound_min", "bound_max"), _valid_prefix_bounds(b, h, s_q, count, q.device)))
-    return attention(q, k, v, scale=scale, causal=causal, **bounds)
+    return _joint(q, image_k, image_v, text_k, text_v, scale, causal, text_valid_len,
+                  image_k.shape[2])
 
 
 def joint_ulysses_attention(q_img, q_txt, image_k, image_v, text_k, text_v, *, scale: float,
@@ -133,14 +157,7 @@ def joint_ulysses_attention(q_img, q_txt, image_k, image_v, text_k, text_v, *, s
     """cp = 1: full joint attention of [q_img | q_txt] over [image | text] keys, split back."""
     _require_cp1("joint_ulysses_attention")
     q = torch.cat([q_img, q_txt], dim=2)
-    k = torch.cat([image_k, text_k], dim=2)
-    v = torch.cat([image_v, text_v], dim=2)
-    bounds = {}
-    if key_valid_len is not None:
-        b, h, s_q, _ = q.shape
-        bounds = dict(zip(("bound_min", "bound_max"),
-                          _valid_prefix_bounds(b, h, s_q, key_valid_len, q.device)))
-    out = attention(q, k, v, scale=scale, causal=causal, **bounds)
+    out = _joint(q, image_k, image_v, text_k, text_v, scale, causal, key_valid_len, 0)
     s_img = q_img.shape[2]
     return out[:, :, :s_img], out[:, :, s_img:]
 

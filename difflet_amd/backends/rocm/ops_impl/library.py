@@ -39,6 +39,20 @@ def _(q, k, v, scale, causal, attention_mask, bound_min, bound_max):
     return q.new_empty((*q.shape[:-1], v.shape[-1]), dtype=v.dtype)
 
 
+@torch.library.custom_op("difflet_rocm::attention_joint", mutates_args=())
+def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
+                    key_count: Optional[Tensor], count_offset: int) -> Tensor:
+    """difflet_rocm_attention_joint: (B, H, S, 128) q over the keys [k | k2], the first
+    key_count[b] + count_offset of them when key_count is given."""
+    return kernels.attention_joint(q, k, v, k2, v2, scale=scale, key_count=key_count,
+                                   count_offset=count_offset)
+
+
+@attention_joint.register_fake
+def _(q, k, v, k2, v2, scale, key_count, count_offset):
+    return q.new_empty(q.shape)
+
+
 # ------------------------------------------------------------------------------------- linear
 #: up to this many input rows a linear runs on the GEMV kernel (HBM-bound on the weight)
 GEMV_ROWS = 8

@@ -5,8 +5,9 @@
 //
 // Work split: a 256-thread workgroup (4 wavefronts) owns 128 query rows of one (batch, head);
 // each wavefront owns 32 of them. K/V stream through LDS in tiles of 64 keys, double-buffered.
-// Unmasked attention over more than 1024 keys runs the ping-pong variant (attn_pp_kernel,
-// below): 8 wavefronts, 256 queries, two groups alternating MFMA and softmax phases.
+// Attention over more than 1024 keys without a mask tensor or causal mask runs the ping-pong
+// variant (attn_pp_kernel, below): 8 wavefronts, 256 queries, two groups alternating MFMA and
+// softmax phases.
 //
 // Operand roles. Scores are computed transposed, S^T = K Q^T (MFMA 32x32x16, first operand a K
 // fragment, second a Q fragment held in registers for the whole kernel), so accumulator lane l
@@ -33,6 +34,8 @@
 // Masking follows the reference: masked scores become the lowest finite float (so a fully
 // masked row averages V, as softmax over equal finfo.min scores does); keys past seq_k do not
 // exist and take -inf.
+#include <limits.h>
+
 #include <mutex>
 #include <vector>
 #include <type_traits>
@@ -74,6 +77,12 @@ struct AttnArgs {
   const int32_t* bmin;
   const int32_t* bmax;
   int64_t bs[3];
+  // second key segment of joint attention: seq_k1 keys in the first, whose tiles end at j1 (a
+  // multiple of the tile; INT_MAX: no second segment), key_tiles in both; boff is added to bmax
+  const uint8_t* k2;
+  const uint8_t* v2;
+  int64_t ks2[3], vs2[3];
+  int seq_k1, j1, key_tiles, boff;
   // split schedule of the ping-pong kernel (sp.groups == 0: one query tile per workgroup)
   AttPlan sp;
   uint8_t* ws;
@@ -471,7 +480,18 @@ __device__ __forceinline__ void vm_phase_barrier() {
   asm volatile("s_barrier" ::: "memory");
 }
 
-template <typename T>
+// GEN: the keys carry a window per query (bound_min / bound_max) or come in two segments (joint
+// attention's [image | text], each in its own tensor: concatenating them first moved 2 x 44 MB
+// at Qwen-Image's 24 x 6889 + 256 keys, 117 us of copies). The segments are tiled separately, so a key
+// tile lies in one of them and its loads pick that segment's buffer with a scalar select; the
+// first segment's last tile and the second's mask their missing rows as the last tile does. A
+// tile inside every window of the wave runs the plain softmax; the others compare each key.
+// Masked keys take a raw score of -2^126 / 2^e (2^e <= the scale, at least 1): a power of two,
+// so its product with the scale is exact and finite and a fully masked row's exponentials are
+// all exp2(0): the row averages v. 24 x 6889 queries x 7145 keys: 1473 us for the joint call on
+// the single-group masked kernel, with the copies and the bounds' fills; 558 us here. The
+// plain instance (GEN false) is compiled apart and keeps its registers.
+template <typename T, bool GEN>
 __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
   typedef typename MfmaT<T>::frag frag;
   // one LDS variable (two K tiles, two V tiles, the split flag): with several, the compiler gives
@@ -487,7 +507,7 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
   const int gt = tid & 255;  // thread index within the group
   const int col = lane & 31, g = lane >> 5;
 
-  const int ntiles = (a.seq_k + BLOCK_N - 1) / BLOCK_N;
+  const int ntiles = GEN ? a.key_tiles : (a.seq_k + BLOCK_N - 1) / BLOCK_N;
   // work: one query tile, or (split schedule) the units of this workgroup's lockstep set in the
   // cut part, then its whole tiles (cut parts first: their merges then overlap the whole tiles
   // of other workgroups instead of all landing at the end; 1-2.5 % faster at 24 x 4608 and
@@ -549,8 +569,33 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
       qf[c] = __builtin_bit_cast(frag, buf_load16(rq, (uint32_t)(my_q * qrow) + (c * 16 + g * 8) * 2));
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   };
-  const i32x4_t rk = rsrc_words(kp, (uint32_t)min((int64_t)a.seq_k * krow, (int64_t)0xffffffff));
-  const i32x4_t rv = rsrc_words(vp, (uint32_t)min((int64_t)a.seq_k * vrow, (int64_t)0xffffffff));
+  const int len1 = GEN ? a.seq_k1 : a.seq_k;  // rows of the (first) segment
+  const i32x4_t rk = rsrc_words(kp, (uint32_t)min((int64_t)len1 * krow, (int64_t)0xffffffff));
+  const i32x4_t rv = rsrc_words(vp, (uint32_t)min((int64_t)len1 * vrow, (int64_t)0xffffffff));
+  // GEN: the second segment's buffer of this group's operand, and the queries' key windows
+  i32x4_t r2 = {};
+  uint32_t row_bytes2 = 0;
+  int lo = 0, hi = INT_MAX, wave_lo = 0, wave_hi = INT_MAX;
+  if constexpr (GEN) {
+    const int64_t row2 = (grp_a ? a.vs2[2] : a.ks2[2]) * 2;
+    const uint8_t* p2 = grp_a ? a.v2 + (b * a.vs2[0] + h * a.vs2[1]) * 2
+                              : a.k2 + (b * a.ks2[0] + h * a.ks2[1]) * 2;
+    r2 = rsrc_words(p2, (uint32_t)min((int64_t)(a.seq_k - len1) * row2, (int64_t)0xffffffff));
+    row_bytes2 = (uint32_t)row2;
+    if (a.bmax && my_q < a.seq_q) {
+      const int64_t bo = b * a.bs[0] + h * a.bs[1] + (int64_t)my_q * a.bs[2];
+      lo = a.bmin ? a.bmin[bo] : 0;
+      hi = a.bmax[bo] + a.boff;
+    }
+    wave_lo = lo, wave_hi = hi;  // the window all of the wave's queries share
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      wave_lo = max(wave_lo, __shfl_xor(wave_lo, o, kWave));
+      wave_hi = min(wave_hi, __shfl_xor(wave_hi, o, kWave));
+    }
+    wave_lo = __builtin_amdgcn_readfirstlane(wave_lo);
+    wave_hi = __builtin_amdgcn_readfirstlane(wave_hi);
+  }
 
   // staging by direct-to-LDS loads, 4 waves per tile: group B loads K, group A loads V. A tile
   // of P slots per row is P instructions of 1 KB; wave wb of the group issues instructions
@@ -568,21 +613,25 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
     const int sl = (wb + 4 * i) * 64 + lane;
     rc[i] = ((uint32_t)(sl / pslots) << 16) | (uint32_t)(min(sl % pslots, 15) * 16);
   }
-  auto dma_voff = [&](int j0, int i) {
-    const uint32_t row = (uint32_t)min(j0 + (int)(rc[i] >> 16), a.seq_k - 1);
-    return row * row_bytes + (rc[i] & 0xffffu);
-  };
-  auto dma_k = [&](int j0, int st) {
+  // this wave's instructions of the key tile at j0, in the segment it lies in
+  auto dma_tile = [&](i32x4_t r, int j0, uint8_t* dst, int slots) {
+    int row0 = j0, last = len1 - 1;
+    uint32_t rb = row_bytes;
+    if (GEN && j0 >= a.j1) {
+      r = r2;
+      rb = row_bytes2;
+      row0 = j0 - a.j1;
+      last = a.seq_k - len1 - 1;
+    }
 #pragma unroll
     for (int i = 0; i < 5; ++i)
-      if (wb + 4 * i < PK_SLOTS)
-        dma16(rk, sk(st) + (wb + 4 * i) * 1024, dma_voff(j0, i));
+      if (wb + 4 * i < slots) {
+        const uint32_t row = (uint32_t)min(row0 + (int)(rc[i] >> 16), last);
+        dma16(r, dst + (wb + 4 * i) * 1024, row * rb + (rc[i] & 0xffffu));
+      }
   };
-  auto dma_v = [&](int j0, int st) {
-#pragma unroll
-    for (int i = 0; i < 5; ++i)
-      dma16(rv, sv(st) + (wb + 4 * i) * 1024, dma_voff(j0, i));
-  };
+  auto dma_k = [&](int j0, int st) { dma_tile(rk, j0, sk(st), PK_SLOTS); };
+  auto dma_v = [&](int j0, int st) { dma_tile(rv, j0, sv(st), PV_SLOTS); };
   // V^T fragment reads: lane l of 16-lane group G supplies key row 4 g + (l >> 2) % 4 of the
   // 8-key half and dims 32 dt + 16 (G % 2) + 4 (l % 4); it receives dim 32 dt + l % 32 of keys
   // {4g .. 4g + 3} (first read) and {8 + 4g .. 8 + 4g + 3} (second), the order of its P values
@@ -596,6 +645,8 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
   uint32_t pp[2][8] = {};  // P of the tile being multiplied next, packed 16-bit pairs
   float m_run = -INFINITY, l_run = 0.f;
   const float cmul = a.scale_log2;
+  // GEN: the raw score of a masked key
+  const float fill = GEN ? -__builtin_ldexpf(1.f, 126 - max(0, __builtin_amdgcn_frexp_expf(cmul))) : 0.f;
 
   // One MFMA phase: O^T += V^T P^T of the tile in sv(vst), 16 MFMAs (steps 0-15: 16-key block
   // gi = step / 4, output dims 32 dt, dt = step % 4, two transposing 8-byte reads each), then
@@ -657,14 +708,29 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
       }
     }
   };
-  auto softmax = [&](int j0) {  // online softmax of s (keys j0 ..), P into pp
-    if (j0 + BLOCK_N > a.seq_k) {  // last tile: keys past seq_k do not exist
+  auto softmax = [&](int j0) {  // online softmax of s (key tile at j0), P into pp
+    int end = a.seq_k;  // keys past the end (of the tile's segment) do not exist
+    if constexpr (GEN) {
+      const bool second = j0 >= a.j1;
+      if (second) j0 += len1 - a.j1;  // the tile's first key
+      else end = len1;
+      if (j0 < wave_lo || j0 + BLOCK_N > wave_hi) {
+#pragma unroll
+        for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int key = j0 + kt2 * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
+            if (key < lo || key >= hi) s[kt2][v] = fill;
+          }
+      }
+    }
+    if (j0 + BLOCK_N > end) {  // a segment's last tile
 #pragma unroll
       for (int kt2 = 0; kt2 < 2; ++kt2)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int key = j0 + kt2 * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
-          if (key >= a.seq_k) s[kt2][v] = -INFINITY;
+          if (key >= end) s[kt2][v] = -INFINITY;
         }
     }
     // Lazy rescaling without a max on the common path: the exponentials are taken relative to
@@ -737,18 +803,18 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
     phase_barrier();
     // ring buffers of tiles j, j + 1, j + 2 (rotated, not j % 3: a division the compiler
     // keeps in vector registers)
-    int r0 = 0, r1 = 1, r2 = 2;
+    int r0 = 0, r1 = 1, rn = 2;
     for (int jt = 0; jt < nt; ++jt) {
       const int j0 = k0 + jt * BLOCK_N;
       softmax(j0);             // phase 2j
       vm_phase_barrier<5>();  // V(j) landed, V(j + 1) may be in flight
-      dma_v(j0 + 2 * BLOCK_N, r2);
+      dma_v(j0 + 2 * BLOCK_N, rn);
       __builtin_amdgcn_s_setprio(1);  // phase 2j + 1 (past the last tile the scores read
       mfma_phase(r0, r1);             // an unused K buffer and go unused)
       __builtin_amdgcn_s_setprio(0);
       phase_barrier();
       const int r = r0;
-      r0 = r1, r1 = r2, r2 = r;
+      r0 = r1, r1 = rn, rn = r;
     }
   } else {
     dma_k(k0, 0);
@@ -1085,7 +1151,18 @@ __global__ void att_zero_counters(int* __restrict__ ctr, int n) {
   if (i < n) ctr[i] = 0;
 }
 
-// The body of both attention entry points. clear_counters: zero the workspace's counters on
+// The second key segment of a joint call (seq_k2 > 0) and its per-batch count of attending keys.
+struct AttnSecond {
+  const void* k;
+  const void* v;
+  int64_t seq_k;
+  const int64_t* k_strides;
+  const int64_t* v_strides;
+  const int32_t* key_count;
+  int64_t count_offset;
+};
+
+// The body of the attention entry points. clear_counters: zero the workspace's counters on
 // the stream before a split-schedule launch (the caller-owned workspace is zeroed once by its
 // owner and left zeroed by the kernels; the library's own scratch is cleared every time).
 static int attention_impl(const char* name, const void* q, const void* k, const void* v,
@@ -1096,7 +1173,7 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
                           int mask_dtype, const int64_t* mask_strides, const int32_t* bound_min,
                           const int32_t* bound_max, const int64_t* bound_strides,
                           void* workspace, int64_t workspace_bytes, bool clear_counters,
-                          difflet_stream_t stream) {
+                          difflet_stream_t stream, const AttnSecond* second = nullptr) {
   DLT_REQUIRE(q && k && v && o && q_strides && k_strides && v_strides && o_strides,
               DIFFLET_EINVAL, "attention: null pointer");
   DLT_REQUIRE(dtype == DIFFLET_BF16 || dtype == DIFFLET_F16 || dtype == DIFFLET_F32,
@@ -1149,9 +1226,12 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   args.seq_k = (int)seq_k;
   // the fast paths need scale > 0 (scores stay raw and are scaled inside exp2); the ping-pong
   // kernel pays a few tiles of pipeline fill, so short key sequences (cross-attention to text)
-  // run the single-group kernel
+  // run the single-group kernel (attention_joint always runs the ping-pong kernel: the other one
+  // reads one segment)
   const bool masked = causal || mask || bound_min || !(scale > 0.0f);
-  const bool pingpong = head_dim == HD && !masked && seq_k > 1024;
+  const bool bounded = bound_min && !causal && scale > 0.0f;
+  const bool gen = second || bounded;  // the ping-pong kernel's instance for windows and segments
+  const bool pingpong = second || (head_dim == HD && (!masked || bounded) && seq_k > 1024);
   const int qblock = pingpong ? 2 * BLOCK_M : BLOCK_M;  // queries per workgroup
   args.q_tiles = (int)((seq_q + qblock - 1) / qblock);
   const int64_t total = (int64_t)args.q_tiles * batch * heads;
@@ -1167,6 +1247,25 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   args.bmax = bound_max;
   if (bound_min)
     for (int i = 0; i < 3; ++i) args.bs[i] = bound_strides[i];
+  args.key_tiles = (int)((seq_k + BLOCK_N - 1) / BLOCK_N);
+  args.seq_k1 = (int)seq_k;
+  args.j1 = INT_MAX;
+  if (second) {
+    args.bmax = second->key_count;
+    args.bs[0] = 1;
+    args.boff = (int)second->count_offset;
+    if (second->seq_k > 0) {
+      args.seq_k = (int)(seq_k + second->seq_k);
+      args.k2 = (const uint8_t*)second->k;
+      args.v2 = (const uint8_t*)second->v;
+      for (int i = 0; i < 3; ++i) {
+        args.ks2[i] = second->k_strides[i];
+        args.vs2[i] = second->v_strides[i];
+      }
+      args.j1 = args.key_tiles * BLOCK_N;
+      args.key_tiles += (int)((second->seq_k + BLOCK_N - 1) / BLOCK_N);
+    }
+  }
   hipStream_t s = (hipStream_t)stream;
   if (dtype == DIFFLET_F32) {
     const int cus = att_device_cus();
@@ -1187,7 +1286,7 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   if (pingpong && workspace) {
     // split schedule when the last wave of workgroups would leave > 10 % of the CUs idle
     const int cus = att_device_cus();
-    args.sp = att_plan(total, (int)((seq_k + BLOCK_N - 1) / BLOCK_N), cus, workspace_bytes);
+    args.sp = att_plan(total, args.key_tiles, cus, workspace_bytes);
     if (args.sp.groups) {
       args.ws = (uint8_t*)workspace;
       grid = dim3((unsigned)cus);
@@ -1209,11 +1308,13 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   using D64 = std::integral_constant<int, 64>;
   using D128 = std::integral_constant<int, 128>;
   if (dtype == DIFFLET_BF16) {
-    if (pingpong) hipLaunchKernelGGL((attn_pp_kernel<bf16>), grid, dim3(512), 0, s, args);
+    if (pingpong && gen) hipLaunchKernelGGL((attn_pp_kernel<bf16, true>), grid, dim3(512), 0, s, args);
+    else if (pingpong) hipLaunchKernelGGL((attn_pp_kernel<bf16, false>), grid, dim3(512), 0, s, args);
     else if (head_dim == 64) fwd(bf16{}, D64{});
     else fwd(bf16{}, D128{});
   } else {
-    if (pingpong) hipLaunchKernelGGL((attn_pp_kernel<f16>), grid, dim3(512), 0, s, args);
+    if (pingpong && gen) hipLaunchKernelGGL((attn_pp_kernel<f16, true>), grid, dim3(512), 0, s, args);
+    else if (pingpong) hipLaunchKernelGGL((attn_pp_kernel<f16, false>), grid, dim3(512), 0, s, args);
     else if (head_dim == 64) fwd(f16{}, D64{});
     else fwd(f16{}, D128{});
   }
@@ -1234,6 +1335,42 @@ extern "C" int difflet_rocm_attention(const void* q, const void* k, const void* 
                         q_strides, k_strides, v_strides, o_strides, scale, causal, mask,
                         mask_dtype, mask_strides, bound_min, bound_max, bound_strides, workspace,
                         workspace_bytes, false, stream);
+}
+
+extern "C" int difflet_rocm_attention_joint(
+    const void* q, const void* k, const void* v, const void* k2, const void* v2, void* o, int dtype,
+    int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_k, int64_t seq_k2, int64_t head_dim,
+    const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+    const int64_t* k2_strides, const int64_t* v2_strides, const int64_t* o_strides, float scale,
+    const int32_t* key_count, int64_t count_offset, void* workspace, int64_t workspace_bytes,
+    difflet_stream_t stream) {
+  DLT_REQUIRE(dtype == DIFFLET_BF16 || dtype == DIFFLET_F16, DIFFLET_EUNSUPPORTED,
+              "attention_joint: dtype %d unsupported (bf16, fp16)", dtype);
+  DLT_REQUIRE(head_dim == HD, DIFFLET_EUNSUPPORTED,
+              "attention_joint: head_dim %lld unsupported (128)", (long long)head_dim);
+  DLT_REQUIRE(scale > 0.0f, DIFFLET_EUNSUPPORTED, "attention_joint: scale must be positive");
+  DLT_REQUIRE(seq_k2 >= 0 && seq_k2 < (1 << 24) && seq_k >= 0 && seq_k + seq_k2 < (1 << 24),
+              DIFFLET_EINVAL, "attention_joint: bad key counts");
+  DLT_REQUIRE(count_offset >= 0 && count_offset < (1 << 24), DIFFLET_EINVAL,
+              "attention_joint: bad count offset");
+  if (seq_k2 > 0) {
+    DLT_REQUIRE(k2 && v2 && k2_strides && v2_strides, DIFFLET_EINVAL,
+                "attention_joint: null pointer");
+    const int64_t* ss[2] = {k2_strides, v2_strides};
+    const void* ps[2] = {k2, v2};
+    for (int i = 0; i < 2; ++i) {
+      DLT_REQUIRE(ss[i][2] % 8 == 0 && ss[i][1] % 8 == 0 && ss[i][0] % 8 == 0 &&
+                      ((uintptr_t)ps[i] & 15) == 0,
+                  DIFFLET_EINVAL, "attention_joint: rows must be 16-byte aligned");
+      DLT_REQUIRE((seq_k2 + 128) * ss[i][2] * 2 < (1LL << 32), DIFFLET_EUNSUPPORTED,
+                  "attention_joint: one head's sequence exceeds 4 GiB");
+    }
+  }
+  const AttnSecond second = {k2, v2, seq_k2, k2_strides, v2_strides, key_count, count_offset};
+  return attention_impl("attention_joint", q, k, v, o, dtype, batch, heads, seq_q, seq_k, head_dim,
+                        q_strides, k_strides, v_strides, o_strides, scale, 0, nullptr, 0, nullptr,
+                        nullptr, nullptr, nullptr, workspace, workspace_bytes, false, stream,
+                        &second);
 }
 
 // ---- attention that allocates nothing: the split schedule's workspace is this file's static

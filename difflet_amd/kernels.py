@@ -151,6 +151,41 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float
     return out
 
 
+def attention_joint(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k2: torch.Tensor,
+                    v2: torch.Tensor, *, scale: float, key_count: torch.Tensor | None = None,
+                    count_offset: int = 0) -> torch.Tensor:
+    """Attention of q [B, H, S, 128] to the keys [k | k2] (values [v | v2]), bf16 or fp16 and
+    scale > 0, without concatenating them. key_count: int32 [B]; keys [0, key_count[b] +
+    count_offset) attend. Segments whose rows the kernel cannot address where they lie (16-byte
+    alignment, 32-bit offsets within a head) are copied first, as concatenating would."""
+    dev = _on_gpu(q, k, v, k2, v2, key_count)
+    b, h, sq, d = q.shape
+    s1, s2 = k.shape[2], k2.shape[2]
+    for t, s in ((k, s1), (v, s1), (k2, s2), (v2, s2)):
+        if t.dtype != q.dtype or t.shape != (b, h, s, d):
+            raise ValueError("attention_joint: q, k, v, k2, v2 differ in dtype or shape")
+    if key_count is not None and (key_count.dtype != torch.int32 or key_count.shape != (b,)):
+        raise ValueError("attention_joint: key_count must be int32 [batch]")
+
+    def addressable(t):
+        st = t.stride()
+        ok = (st[3] == 1 and all(x % 8 == 0 for x in st[:3]) and t.data_ptr() % 16 == 0
+              and (t.shape[2] + 128) * st[2] * 2 < 1 << 32)
+        return t if ok else t.clone(memory_format=torch.contiguous_format)
+
+    k, v, k2, v2 = (addressable(t) for t in (k, v, k2, v2))
+    q = q if q.stride(-1) == 1 else q.contiguous()
+    key_count = None if key_count is None else key_count.contiguous()
+    out = torch.empty((b, h, sq, d), dtype=v.dtype, device=dev)
+    workspace = attention_workspace(dev)
+    st = lib().difflet_rocm_attention_joint(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(k2), _ptr(v2), _ptr(out), _dt(q), b, h, sq, s1, s2, d,
+        *(_arr(t.stride()[:3]) for t in (q, k, v, k2, v2, out)), float(scale), _ptr(key_count),
+        int(count_offset), _ptr(workspace), workspace.numel(), _stream(dev))
+    check(st, "attention_joint")
+    return out
+
+
 # ------------------------------------------------------------------------------------ GEMM
 class Problem:
     """One problem of a grouped GEMM: C = epilogue(A W^T + bias)."""

@@ -61,8 +61,8 @@ int difflet_rocm_device_count(void);
  * bound_max: optional int32 [batch, heads, seq_q] through strides; keys in [min, max) attend
  * (difflet/backends/cpu/ops_impl/attention.py:24-35). Masked scores take the dtype's lowest
  * finite value, so a fully masked row averages v exactly as the reference does.
- * workspace / workspace_bytes: optional device memory for the split schedule of unmasked
- * attention over more than 1024 keys. When the launch's 256-query tiles would leave the last
+ * workspace / workspace_bytes: optional device memory for the split schedule of attention,
+ * unmasked or with bounds, over more than 1024 keys. When the launch's 256-query tiles would leave the last
  * wave of workgroups under 90 % full, one workgroup per compute unit runs the last round's
  * query tiles cut along the keys over lockstep sets of workgroups (the workgroups of a set read
  * the same key tiles together), then the full rounds of whole tiles; query tiles cut
@@ -79,6 +79,21 @@ int difflet_rocm_attention(const void* q, const void* k, const void* v, void* o,
                            const int64_t* mask_strides, const int32_t* bound_min,
                            const int32_t* bound_max, const int64_t* bound_strides,
                            void* workspace, int64_t workspace_bytes, difflet_stream_t stream);
+
+/* Joint attention whose keys come in two segments, [k | k2] and [v | v2] (the cp = 1 forms of
+ * difflet/backends/cpu/ops_impl/attention.py:55-143): difflet_rocm_attention on the concatenated
+ * keys, which are never materialized. k2, v2: [batch, heads, seq_k2, head_dim] through strides
+ * (seq_k2 0: none). key_count: optional int32 [batch]; keys [0, key_count[b] + count_offset) of
+ * the concatenation attend, the others are masked as bound_max masks them. BF16 or F16,
+ * head_dim 128, scale > 0, seq_k > 0; the workspace is difflet_rocm_attention's. */
+int difflet_rocm_attention_joint(const void* q, const void* k, const void* v, const void* k2,
+                                 const void* v2, void* o, int dtype, int64_t batch, int64_t heads,
+                                 int64_t seq_q, int64_t seq_k, int64_t seq_k2, int64_t head_dim,
+                                 const int64_t* q_strides, const int64_t* k_strides,
+                                 const int64_t* v_strides, const int64_t* k2_strides,
+                                 const int64_t* v2_strides, const int64_t* o_strides, float scale,
+                                 const int32_t* key_count, int64_t count_offset, void* workspace,
+                                 int64_t workspace_bytes, difflet_stream_t stream);
 
 /* Bytes of attention workspace the split schedule needs on the current device: 16 KiB of
  * counters + 2 x 132 KiB per compute unit (0 without a device). No counterpart in the
