@@ -77,7 +77,7 @@ def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> T
         x = F.pad(x, (0, k_pad - kx))
     if bias is not None and bias.shape[0] != n_pad:
         bias = F.pad(bias, (0, n_pad - bias.shape[0]))
-    y = kernels.linear(x if x.stride(-1) == 1 else x.contiguous(), w, bias)
+    y = kernels.linear(x if x.stride(-1) == 1 else x.contiguous(), w, bias, workspace="call")
     return y if n_pad == out_features else y[:, :out_features].contiguous()
 
 
@@ -118,7 +118,7 @@ def fp8_linear(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tens
     else:
         aq, asc = kernels.quantize_fp8_rowwise(x)
     kernels.gemm_grouped([kernels.Problem(aq, w_kernel, y, bias, a_scale=asc, w_scale=w_scale)],
-                         kind="mx" if mx else "fp8")
+                         kind="mx" if mx else "fp8", workspace="call")
     return y
 
 

@@ -22,7 +22,7 @@ REPO = PKG.parent
 LIB_NAME = "libdifflet_rocm.so"
 LIB_PATH = PKG / LIB_NAME
 OBJ_DIR = REPO / "_build" / "difflet_rocm"
-SOURCES = ("runtime.hip", "elementwise.hip", "gemm.hip", "gemm_f32.hip", "attention.hip",
+SOURCES = ("runtime.hip", "elementwise.hip", "gemm.hip", "gemm_small.hip", "gemm_f32.hip", "attention.hip",
            "quant.hip", "vae.hip", "conv.hip")
 ARCH = "gfx950"
 

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "gemm_small.hpp"
 
 namespace dlt {
 
@@ -1056,6 +1057,30 @@ static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes) {
   return pl;
 }
 
+template <Elem E> constexpr SmallElem small_elem() {
+  return E == Elem::BF16 ? SmallElem::BF16 : E == Elem::FP8 ? SmallElem::FP8 : SmallElem::MX;
+}
+// The small-launch plan of one problem, weighed against the time of the 256 x 256 tiles that
+// `sk` schedules: about 1.35 us (fp8 and MX 1.05) per K stage with few units busy, 1.65 with all
+// of them, and for a split launch 1.6 per stage of the longest range plus 40 for the partial sums
+// (measured within 10 % at 24 to 288 tiles).
+template <Elem E>
+static SmallPlan small_plan_of(int64_t m, int64_t n, int64_t k, int64_t scratch, const SkPlan& sk) {
+  const int cus = device_cus();
+  if (cus <= 0) return SmallPlan{0, 0, 0, 0};
+  const int64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
+  const int nk = (int)(k / ElemTraits<E>::KT);
+  double us = 0;
+  if (sk.groups > 0) {
+    us = ((double)(sk.dp / cus) * nk + (double)sk.units / sk.nx * sk.gran) * 1.6 + 40.0;
+  } else {
+    const double fill = std::min(1.0, (double)tiles / cus);
+    us = (double)((tiles + cus - 1) / cus) *
+         (nk * (E == Elem::BF16 ? 1.35 + 0.3 * fill : 1.05 + 0.5 * fill) + 5.0);
+  }
+  return small_plan(small_elem<E>(), m, n, k, cus, scratch, us);
+}
+
 template <Elem E>
 static int gemm_launch(const char* name, int nproblems, const difflet_gemm_problem* problems,
                        int64_t n, int64_t k, int epilogue, int64_t act_col_start,
@@ -1197,6 +1222,19 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
   }
   args.sk = sk_plan((int)tiles, (int)(k / KT), E == Elem::MX ? 4 : 1,
                     workspace ? device_cus() : 0, workspace ? workspace_bytes : 0);
+  // launches of few tiles: smaller tiles, K cut into pieces (gemm_small.hip)
+  if (nproblems == 1 && !qk &&
+      (epilogue == DIFFLET_EPI_NONE || epilogue == DIFFLET_EPI_GATE_RESIDUAL)) {
+    const SmallPlan plan =
+        small_plan_of<E>(problems[0].m, n, k, workspace ? workspace_bytes - SK_CTR_BYTES : 0,
+                         args.sk);
+    if (plan.bm > 0) {
+      gemm_small(small_elem<E>(), plan, problems[0], n, k, epilogue == DIFFLET_EPI_GATE_RESIDUAL,
+                 args.p[0].rows_per_batch, workspace ? (uint8_t*)workspace + SK_CTR_BYTES : nullptr,
+                 stream);
+      return dlt_check_launch(name);
+    }
+  }
   args.ws = (uint8_t*)workspace;
   constexpr int NT = ElemTraits<E>::WN;
   dim3 grid((unsigned)(args.sk.dp + args.sk.groups)), block(128 * NT);
@@ -1245,6 +1283,17 @@ using namespace dlt;
 extern "C" int64_t difflet_rocm_gemm_workspace_bytes(void) {
   const int cus = device_cus();
   return cus > 0 ? sk_workspace_bytes(cus) : 0;
+}
+
+extern "C" int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0 || m >= (1LL << 30) || n >= (1LL << 30) || k >= (1LL << 30))
+    return 0;
+  constexpr int64_t cap = 64LL << 20;
+  const SkPlan whole = {};
+  const SmallPlan p = kind == 0   ? small_plan_of<Elem::BF16>(m, n, k, cap, whole)
+                      : kind == 1 ? small_plan_of<Elem::FP8>(m, n, k, cap, whole)
+                                  : small_plan_of<Elem::MX>(m, n, k, cap, whole);
+  return p.pieces > 1 ? SK_CTR_BYTES + p.pieces * m * n * 4 : 0;
 }
 
 extern "C" int difflet_rocm_gemm_bf16(int nproblems, const difflet_gemm_problem* problems,

@@ -222,6 +222,7 @@ class QkNormRope:
 
 _GEMM_FN = {"bf16": "difflet_rocm_gemm_bf16", "fp8": "difflet_rocm_gemm_fp8_rowwise",
             "mx": "difflet_rocm_gemm_mxfp8"}
+_KIND_ID = {"bf16": 0, "fp8": 1, "mx": 2}
 
 
 _WORKSPACE: dict[tuple[int, int], torch.Tensor] = {}
@@ -332,8 +333,10 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
                  workspace: torch.Tensor | None | str = None,
                  qk: QkNormRope | None = None) -> None:
     """Runs up to 4 GEMMs sharing N, K and the epilogue in one launch (writes each p.c).
-    workspace: None (every tile whole on one workgroup, the default), "shared" (the current
-    stream's, see gemm_workspace) or a zero-filled uint8 tensor of
+    workspace: None (every tile whole on one workgroup, the default), "call" (scratch of this
+    call alone, from torch's allocator, where a launch of few tiles gains by cutting K: safe on
+    any stream and under graph capture), "shared" (the current stream's, see gemm_workspace) or
+    a zero-filled uint8 tensor of
     difflet_rocm_gemm_workspace_bytes() bytes, which lets a launch whose last wave of tiles
     would be poorly filled cut those tiles along K over the XCDs when that takes a quarter and
     at least 24 K stages off its time (Qwen-Image's 336-tile projections, Wan's bf16 text k/v
@@ -401,9 +404,18 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
             q.norm_k = p.norm_k.data_ptr() if p.norm_k is not None else None
             q.rope_row0 = int(p.rope_row0)
     if isinstance(workspace, str):
-        if workspace != "shared":
-            raise ValueError(f"workspace must be 'shared', a tensor or None, got {workspace!r}")
-        workspace = gemm_workspace(dev)
+        if workspace == "shared":
+            workspace = gemm_workspace(dev)
+        elif workspace == "call":
+            workspace = None
+            if len(problems) == 1 and qk is None and epilogue in (_lib.EPI_NONE,
+                                                                  _lib.EPI_GATE_RESIDUAL):
+                nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID[kind], arr[0].m, n, k)
+                if nbytes:
+                    workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        else:
+            raise ValueError("workspace must be 'shared', 'call', a tensor or None, "
+                             f"got {workspace!r}")
     ws_ptr, ws_bytes = (None, 0) if workspace is None else (workspace.data_ptr(),
                                                            workspace.numel())
     qk_arg = None
@@ -421,7 +433,8 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
            epilogue: int = _lib.EPI_NONE, gate: torch.Tensor | None = None,
            residual: torch.Tensor | None = None, act_col_start: int = 0,
-           rows_per_batch: int | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+           rows_per_batch: int | None = None, out: torch.Tensor | None = None,
+           workspace: torch.Tensor | None | str = None) -> torch.Tensor:
     """bf16 ``x W^T + b`` over the last dim of x, with an optional fused epilogue."""
     x2 = _rows2d(x, "linear")
     n = w.shape[0]
@@ -429,7 +442,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
                                                 device=x.device)
     res2 = _rows2d(residual, "residual") if residual is not None else None
     gemm_grouped([Problem(x2, w, c, bias, gate, res2, rows_per_batch=rows_per_batch)],
-                 kind="bf16", epilogue=epilogue, act_col_start=act_col_start)
+                 kind="bf16", epilogue=epilogue, act_col_start=act_col_start, workspace=workspace)
     return c.reshape(*x.shape[:-1], n) if out is None else c
 
 

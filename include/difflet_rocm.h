@@ -210,12 +210,23 @@ typedef struct difflet_gemm_qk {
  * eighth, stay whole, and so does an MXFP8 projection of 512 rows at K = 4096). The workgroup
  * finishing a cut tile adds the fp32 partial sums of the others in a fixed order, so results
  * are deterministic for a given device. With workspace NULL (or too small) every tile runs
- * whole on one workgroup. The workspace must be zero-filled once when allocated; the GEMMs
+ * whole on one workgroup. A launch of one problem with few tiles (up to 4096 rows, epilogue NONE
+ * or GATE_RESIDUAL, no fused q/k norm) runs in smaller tiles instead, and with a workspace of
+ * difflet_rocm_gemm_scratch_bytes or more may cut K into pieces, whose fp32 sums a second kernel
+ * adds in order (nothing in the workspace need be zero for that, and its counters stay as they
+ * are). The workspace must be zero-filled once when allocated; the GEMMs
  * leave it zeroed. Launches that may overlap in time (different streams) must not share one.
  * Returns the bytes needed on the current device: 16 KiB of counters + 2 x 256 KiB per compute
  * unit. No counterpart in the reference, whose linears call the vendor BLAS
  * (torch.nn.functional.linear, difflet/backends/cpu/ops_impl/linear.py:9-41). */
 int64_t difflet_rocm_gemm_workspace_bytes(void);
+
+/* Bytes of scratch with which one m x n x k problem (kind 0 bf16, 1 fp8 per row, 2 MXFP8; epilogue
+ * NONE or GATE_RESIDUAL) runs at its fastest among the small-launch plans: passed as the
+ * workspace, not zeroed, used by that launch only. 0: no scratch helps. Always less than
+ * difflet_rocm_gemm_workspace_bytes, so such a buffer never serves the split schedule, which
+ * needs zeroed counters. */
+int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k);
 
 /* bf16 x bf16 -> fp32 accumulate -> bf16. k % 64 == 0. */
 int difflet_rocm_gemm_bf16(int nproblems, const difflet_gemm_problem* problems, int64_t n,

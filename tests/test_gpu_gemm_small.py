@@ -1,0 +1,72 @@
+"""GEMM launches of few tiles (64-, 128- and 256-row tiles, K whole or cut into pieces): every
+element type and both epilogues at the edges of tiles, K stages and pieces, against the fp32
+reference; scratch full of NaN patterns; strided and 8-byte aligned outputs; graph replays.
+
+Tolerance: the products are exact in fp32 and the output is rounded once to bf16 (relative error
+up to 2^-9, rms below 2^-9): rel L2 < 2^-9 plus 2e-4 for fp32 sums in another order. The gated
+epilogue adds a rounded residual of the same size: the same bound."""
+
+import pytest
+import torch
+
+from difflet_amd import _lib, kernels
+from test_gpu_gemm_split import _operands, _reference, rel_l2, rnd
+
+pytestmark = pytest.mark.gpu
+TOL = 2.0 ** -9 + 2e-4
+
+# (m, n, k): one row tile and its edges, two and three row tiles, narrow and ragged n, one K stage,
+# K that pieces divide unevenly (MXFP8 in units of 4 stages), many column tiles
+SHAPES = [(9, 4, 128), (64, 128, 128), (65, 132, 256), (63, 3076, 3072), (128, 512, 15360),
+          (129, 252, 4096), (200, 3072, 6912), (257, 128, 7808), (512, 5120, 5120),
+          (1024, 3072, 12288), (1500, 5120, 1280), (2047, 3072, 3072), (16, 18432, 3072)]
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "mx"])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_small_gemm_matches_the_reference(gpu, kind, m, n, k):
+    print(f"small gemm {kind} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w, b = rnd(g, m, k), rnd(g, n, k, std=0.05), rnd(g, n, std=0.1)
+    aq, wq, sa, sw = _operands(kind, a, w, gpu)
+    ref = _reference(kind, a, w, b)
+    bg = b.to(gpu)
+    ws = torch.full((96 << 20,), 0xff, dtype=torch.uint8, device=gpu)  # NaN patterns
+    outs = []
+    for workspace in (None, "call", ws):
+        c = torch.full((m, n + 12), float("nan"), dtype=torch.bfloat16, device=gpu)[:, 4:n + 4]
+        kernels.gemm_grouped([kernels.Problem(aq, wq, c, bg, a_scale=sa, w_scale=sw)], kind=kind,
+                             workspace=workspace)
+        outs.append(c)
+        assert rel_l2(c, ref) < TOL
+    assert torch.equal(outs[1], outs[2])  # the plan does not depend on where the scratch lies
+    # gate * (acc + bias) + residual written over the residual
+    res, gate = rnd(g, m, n).to(gpu), rnd(g, 1, n).to(gpu)
+    want = res.float().cpu() + gate.float().cpu() * ref
+    kernels.gemm_grouped([kernels.Problem(aq, wq, res, bg, gate, res, a_scale=sa, w_scale=sw)],
+                         kind=kind, epilogue=_lib.EPI_GATE_RESIDUAL, workspace="call")
+    assert rel_l2(res, want) < TOL
+
+
+def test_small_gemm_in_a_replayed_graph(gpu):
+    """K pieces under capture: scratch from the graph's pool, each replay equal to eager."""
+    from difflet_amd.backends.rocm.ops_impl import library
+
+    g = torch.Generator().manual_seed(5)
+    x, w, b = rnd(g, 128, 12288).to(gpu), rnd(g, 3072, 12288, std=0.05).to(gpu), rnd(g, 3072).to(gpu)
+    assert _lib.load().difflet_rocm_gemm_scratch_bytes(0, 128, 3072, 12288) > 0
+    want = library.linear(x, w, b, 3072)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = library.linear(x, w, b, 3072)
+    for i in range(3):
+        y.zero_()
+        x2 = rnd(g, 128, 12288).to(gpu) if i == 1 else x
+        eager = library.linear(x2, w, b, 3072)
+        if i == 1:
+            x.copy_(x2)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager)
+    assert not torch.equal(y, want)
