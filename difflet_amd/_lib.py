@@ -74,6 +74,9 @@ SIGNATURES: dict[str, tuple] = {
     "difflet_rocm_attention_joint": (_i32, [
         _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64,
         _i64p, _i64p, _i64p, _i64p, _i64p, _i64p, _f32, _vp, _i64, _vp, _i64, _vp]),
+    "difflet_rocm_attention_relative_bias": (_i32, [
+        _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64,
+        _i64p, _i64p, _i64p, _i64p, _f32, _vp, _i64, _vp, _i64, _vp]),
     "difflet_rocm_attention_workspace_bytes": (_i64, []),
     "difflet_rocm_attention_noalloc": (_i32, [
         _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64,

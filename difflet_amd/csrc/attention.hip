@@ -83,6 +83,12 @@ struct AttnArgs {
   const uint8_t* v2;
   int64_t ks2[3], vs2[3];
   int seq_k1, j1, key_tiles, boff;
+  // relative-position bias (MODE 2): diag[h][k - q + seq_q - 1], rows of diag_ld floats, and the
+  // keys that attend, keep[b][k] != 0 (NULL: all)
+  const float* diag;
+  int64_t diag_ld;
+  const uint8_t* keep;
+  int64_t keep_ld;
   // split schedule of the ping-pong kernel (sp.groups == 0: one query tile per workgroup)
   AttPlan sp;
   uint8_t* ws;
@@ -231,8 +237,42 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
+// The relative-position bias of a lane's 32 scores of a key tile, 8 quads of keys: diag is a row
+// of 2 x 512 - 1 floats at a text encoder's 512 tokens, so the loads hit the cache where the
+// [heads, 512, 512] table the row expands to is 67 MB, written once (56 us) and read by every
+// layer's attention (84 us a layer; 21 here). rd's range ends with the row; the offset of
+// a query past seq_q wraps below zero and reads zero.
+struct RelBias {
+  f32x4 v[2][4];
+  uint64_t kept;  // the tile's attending keys, bit = key - j0
+  __device__ __forceinline__ void load(const AttnArgs& a, __amdgpu_buffer_rsrc_t rd, int b, int q,
+                                       int j0, int lane) {
+    const int g = lane >> 5;
+#pragma unroll
+    for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[kt2][u] = __builtin_bit_cast(
+            f32x4, buf_load16(rd, (uint32_t)(j0 + kt2 * 32 + u * 8 + g * 4 - q + a.seq_q - 1) * 4u));
+    kept = ~0ull;
+    if (a.keep) {
+      const int key = j0 + lane;
+      kept = __ballot(key < a.seq_k && a.keep[b * a.keep_ld + key] != 0);
+    }
+  }
+  // bit of score (kt2, r) of a lane in group g
+  __device__ __forceinline__ bool keeps(int kt2, int r, int g) const {
+    const uint32_t half = (uint32_t)(kept >> (32 * kt2)) >> (4 * g);
+    return (half >> ((r >> 2) * 8 + (r & 3))) & 1u;
+  }
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t diag_rsrc(const AttnArgs& a, int h) {
+  return make_rsrc(a.diag + h * a.diag_ld, (uint32_t)(a.diag_ld * 4));
+}
+
 // D: head dim, 128 or 64 (T5 / UMT5 encoders). The K tile's row pitch is D * 2 + 16 bytes.
-template <typename T, bool MASKED, int D>
+// MODE: 0 plain, 1 masks / bounds / causal, 2 relative-position bias and key padding.
+template <typename T, int MODE, int D>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs a) {
   typedef typename MfmaT<T>::frag frag;
   constexpr int KP = D * 2 + 16;      // K row pitch
@@ -322,12 +362,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs a) {
   float m_run = -INFINITY, l_run = 0.f;
 
   int bmin = 0, bmax = a.seq_k;
-  if (MASKED && a.bmin && my_q < a.seq_q) {
+  if (MODE == 1 && a.bmin && my_q < a.seq_q) {
     bmin = a.bmin[b * a.bs[0] + h * a.bs[1] + (int64_t)my_q * a.bs[2]];
     bmax = a.bmax[b * a.bs[0] + h * a.bs[1] + (int64_t)my_q * a.bs[2]];
   }
 
   const int ntiles = (a.seq_k + BLOCK_N - 1) / BLOCK_N;
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t rdiag = rk;
+  if constexpr (MODE == 2) rdiag = diag_rsrc(a, h);
   load_tile(0);
   store_tile(0);
   __syncthreads();
@@ -335,6 +377,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs a) {
   for (int jt = 0; jt < ntiles; ++jt) {
     const int st = jt & 1;
     const int j0 = jt * BLOCK_N;
+    [[maybe_unused]] RelBias rb;  // issued ahead of the tile's loads: a wait for it leaves those
+    if constexpr (MODE == 2) rb.load(a, rdiag, b, my_q, j0, lane);
     if (jt + 1 < ntiles) load_tile(j0 + BLOCK_N);
 
     // ---- S^T = K Q^T for 2 x 32 keys
@@ -354,7 +398,22 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs a) {
     // Scores stay raw in the fast path (p = exp2(s * cmul - m)); the masked path scales them
     // first (cmul = 1) so additive masks and finfo.min fills work in scaled units.
     float cmul = a.scale_log2;
-    if (MASKED) {
+    if constexpr (MODE == 2) {
+      cmul = 1.0f;
+#pragma unroll
+      for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          s[kt2][v] = add_mask(s[kt2][v] * a.scale_log2, rb.v[kt2][v >> 2][v & 3], LOG2E);
+      if (rb.kept != ~0ull) {
+#pragma unroll
+        for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (!rb.keeps(kt2, v, g)) s[kt2][v] = -FLT_MAX;
+      }
+    }
+    if (MODE == 1) {
       cmul = 1.0f;
 #pragma unroll
       for (int kt2 = 0; kt2 < 2; ++kt2)
@@ -1050,97 +1109,164 @@ extern "C" int64_t difflet_rocm_attention_workspace_bytes(void) {
   return cus > 0 ? att_workspace_bytes(cus) : 0;
 }
 
-// ---- fp32 inputs (models run in fp32, as the reference's CPU op computes them): scores,
-// softmax and P V in fp32 on the VALU, one query per lane, 256 queries per workgroup (64 when
-// 256 would leave most compute units idle). K and V tiles of 32 keys go through LDS and are read
-// by every lane at the same address (broadcast).
-// Online softmax per lane over each tile; masks, bounds, causal and scale as the MFMA kernels.
-constexpr int F32_TILE = 32;
-template <int D, int NQ>  // NQ: queries (threads) per workgroup, 64 or 256
-__global__ __launch_bounds__(NQ, 1) void attn_f32_kernel(const AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float skk[F32_TILE][D];
-  __shared__ __attribute__((aligned(16))) float svv[F32_TILE][D];
-  const int tid = threadIdx.x;
+// ---- fp32 inputs (models run in fp32, as the reference's CPU op computes them): scores, softmax
+// and P V in fp32, on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), with the work split and
+// operand roles of attn_fwd_kernel: 4 wavefronts of 32 queries, tiles of 64 keys, S^T = K Q^T and
+// O^T += V^T P^T, so that P never leaves registers. An MFMA sums two k values, one per lane
+// group: step (c, e) of the scores takes dim 8 c + 4 g + e (one 16-byte LDS read of K feeds four
+// steps), step (kt2, v) of P V the two keys whose probabilities the groups hold in register v. V
+// is read 4 bytes per lane from row-major rows of D + 8 floats, which puts the groups' rows, 4
+// keys apart, in opposite halves of the banks. One K/V tile in LDS, the next in registers.
+// It replaces one query per lane on the VALU, whose dot products were serial chains of D FMAs:
+// 2 x 64 heads x 226 tokens of dim 64 with bias and padding 315 -> 31 us.
+template <int D, int MODE>
+__global__ __launch_bounds__(256, 1) void attn_f32_kernel(const AttnArgs a) {
+  constexpr int KP = D + 4, VP = D + 8;  // row pitches in floats
+  constexpr int NDT = D / 32, R4 = BLOCK_N * D / 4 / 256;  // 16-byte pieces per thread and tile
+  __shared__ __attribute__((aligned(16))) float sk[BLOCK_N * KP];
+  __shared__ __attribute__((aligned(16))) float sv[BLOCK_N * VP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 31, g = lane >> 5;
   const int bh = blockIdx.x / a.q_tiles, qt = blockIdx.x % a.q_tiles;
   const int b = bh / a.heads, h = bh % a.heads;
-  const int my_q = qt * NQ + tid;
+  const int my_q = qt * BLOCK_M + wave * 32 + col;
   const bool qok = my_q < a.seq_q;
   const float* qp = reinterpret_cast<const float*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const float* kp = reinterpret_cast<const float*>(a.k) + b * a.ks[0] + h * a.ks[1];
   const float* vp = reinterpret_cast<const float*>(a.v) + b * a.vs[0] + h * a.vs[1];
-  float q[D], o[D];
+
+  f32x4 qf[D / 8];  // dims 8 c + 4 g .. + 4 of row my_q
 #pragma unroll
-  for (int d = 0; d < D; d += 4) {
-    const f32x4 x = qok ? *reinterpret_cast<const f32x4*>(qp + (int64_t)my_q * a.qs[2] + d)
-                        : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < D / 8; ++c)
+    qf[c] = qok ? *reinterpret_cast<const f32x4*>(qp + (int64_t)my_q * a.qs[2] + c * 8 + g * 4)
+                : f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 gk[R4], gv[R4];
+  auto load_tile = [&](int j0) {  // rows past seq_k: zeros (their scores are -inf)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      q[d + e] = x[e];
-      o[d + e] = 0.f;
+    for (int i = 0; i < R4; ++i) {
+      const int x = tid + 256 * i, key = j0 + x / (D / 4), d = (x % (D / 4)) * 4;
+      const bool ok = key < a.seq_k;
+      gk[i] = ok ? *reinterpret_cast<const f32x4*>(kp + (int64_t)key * a.ks[2] + d) : f32x4{};
+      gv[i] = ok ? *reinterpret_cast<const f32x4*>(vp + (int64_t)key * a.vs[2] + d) : f32x4{};
     }
-  }
+  };
+  f32x16 acc[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i) acc[i] = f32x16{};
+  float m_run = -INFINITY, l_run = 0.f;
   int bmin = 0, bmax = a.seq_k;
-  if (a.bmin && qok) {
+  if (MODE == 1 && a.bmin && qok) {
     bmin = a.bmin[b * a.bs[0] + h * a.bs[1] + (int64_t)my_q * a.bs[2]];
     bmax = a.bmax[b * a.bs[0] + h * a.bs[1] + (int64_t)my_q * a.bs[2]];
   }
   const float scale = a.scale_log2 / LOG2E;
-  float m_run = -INFINITY, l_run = 0.f;
-  for (int j0 = 0; j0 < a.seq_k; j0 += F32_TILE) {
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t rdiag = make_rsrc(a.q, 0);
+  if constexpr (MODE == 2) rdiag = diag_rsrc(a, h);
+
+  load_tile(0);
+  for (int j0 = 0; j0 < a.seq_k; j0 += BLOCK_N) {
     __syncthreads();  // the previous tile's reads are done
-    for (int i = tid; i < F32_TILE * D / 4; i += NQ) {
-      const int key = j0 + i / (D / 4), d = (i % (D / 4)) * 4;
-      f32x4 kv = {0.f, 0.f, 0.f, 0.f}, vv = {0.f, 0.f, 0.f, 0.f};
-      if (key < a.seq_k) {
-        kv = *reinterpret_cast<const f32x4*>(kp + (int64_t)key * a.ks[2] + d);
-        vv = *reinterpret_cast<const f32x4*>(vp + (int64_t)key * a.vs[2] + d);
-      }
-      *reinterpret_cast<f32x4*>(&skk[i / (D / 4)][d]) = kv;
-      *reinterpret_cast<f32x4*>(&svv[i / (D / 4)][d]) = vv;
+#pragma unroll
+    for (int i = 0; i < R4; ++i) {
+      const int x = tid + 256 * i, row = x / (D / 4), d = (x % (D / 4)) * 4;
+      *reinterpret_cast<f32x4*>(sk + row * KP + d) = gk[i];
+      *reinterpret_cast<f32x4*>(sv + row * VP + d) = gv[i];
     }
     __syncthreads();
-    float sc[F32_TILE];
-    float mx = -INFINITY;
-#pragma unroll 4
-    for (int j = 0; j < F32_TILE; ++j) {
-      const int key = j0 + j;
-      float dot = 0.f;
+    [[maybe_unused]] RelBias rb;
+    if constexpr (MODE == 2) rb.load(a, rdiag, b, my_q, j0, lane);
+    if (j0 + BLOCK_N < a.seq_k) load_tile(j0 + BLOCK_N);
+
+    f32x16 s[2] = {f32x16{}, f32x16{}};
 #pragma unroll
-      for (int d = 0; d < D; ++d) dot += q[d] * skk[j][d];
-      float x = dot * scale;
-      bool masked = key < bmin || key >= bmax || (a.causal && key > my_q);
-      if (a.mask && !masked && key < a.seq_k && qok) {
-        const int64_t mo = b * a.ms[0] + h * a.ms[1] + (int64_t)my_q * a.ms[2] +
-                           (int64_t)key * a.ms[3];
-        if (a.mask_dtype == DIFFLET_BOOL) masked = reinterpret_cast<const uint8_t*>(a.mask)[mo] == 0;
-        else x = add_mask(x, load_mask(a, mo), 1.0f);
-      }
-      x = masked ? -FLT_MAX : x;
-      if (key >= a.seq_k) x = -INFINITY;  // keys past seq_k do not exist
-      sc[j] = x;
-      mx = fmaxf(mx, x);
+    for (int c = 0; c < D / 8; ++c) {
+      f32x4 kf[2];
+#pragma unroll
+      for (int kt2 = 0; kt2 < 2; ++kt2)
+        kf[kt2] = *reinterpret_cast<const f32x4*>(sk + (kt2 * 32 + col) * KP + c * 8 + g * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int kt2 = 0; kt2 < 2; ++kt2)
+          s[kt2] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kt2][e], qf[c][e], s[kt2], 0, 0, 0);
     }
-    const float m_new = fmaxf(m_run, mx);
+    // scale, bias, masks: scores in natural units
+#pragma unroll
+    for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int key = j0 + kt2 * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
+        float x = s[kt2][v] * scale;
+        if constexpr (MODE == 1) {
+          bool masked = key < bmin || key >= bmax || (a.causal && key > my_q);
+          if (a.mask && !masked && key < a.seq_k && qok) {
+            const int64_t mo = b * a.ms[0] + h * a.ms[1] + (int64_t)my_q * a.ms[2] +
+                               (int64_t)key * a.ms[3];
+            if (a.mask_dtype == DIFFLET_BOOL)
+              masked = reinterpret_cast<const uint8_t*>(a.mask)[mo] == 0;
+            else
+              x = add_mask(x, load_mask(a, mo), 1.0f);
+          }
+          x = masked ? -FLT_MAX : x;
+        }
+        if constexpr (MODE == 2) {
+          x = add_mask(x, rb.v[kt2][v >> 2][v & 3], 1.0f);
+          x = rb.keeps(kt2, v, g) ? x : -FLT_MAX;
+        }
+        s[kt2][v] = x;
+      }
+    if (j0 + BLOCK_N > a.seq_k) {  // last tile: keys past seq_k do not exist
+#pragma unroll
+      for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (j0 + kt2 * 32 + (v >> 2) * 8 + g * 4 + (v & 3) >= a.seq_k) s[kt2][v] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[kt2][v]);
+    const float m_new = fmaxf(m_run, pair_max(mx));
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __expf(m_run - m_use);
     m_run = m_new;
-    l_run *= alpha;
+    float ls = 0.f;
 #pragma unroll
-    for (int d = 0; d < D; ++d) o[d] *= alpha;
-#pragma unroll 4
-    for (int j = 0; j < F32_TILE; ++j) {
-      const float p = __expf(sc[j] - m_use);
-      l_run += p;
+    for (int kt2 = 0; kt2 < 2; ++kt2)
 #pragma unroll
-      for (int d = 0; d < D; ++d) o[d] += p * svv[j][d];
+      for (int v = 0; v < 16; ++v) {
+        s[kt2][v] = __expf(s[kt2][v] - m_use);
+        ls += s[kt2][v];
+      }
+    l_run = l_run * alpha + ls;
+    if (__any(alpha != 1.0f)) {
+#pragma unroll
+      for (int i = 0; i < NDT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][v] *= alpha;
     }
+#pragma unroll
+    for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int key = kt2 * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(sv[key * VP + dt * 32 + col], s[kt2][v],
+                                                         acc[dt], 0, 0, 0);
+      }
   }
+  const float inv = 1.0f / pair_sum(l_run);
   if (qok) {
     float* op = reinterpret_cast<float*>(a.o) + b * a.os[0] + h * a.os[1] + (int64_t)my_q * a.os[2];
-    const float inv = 1.0f / l_run;
 #pragma unroll
-    for (int d = 0; d < D; d += 4)
-      *reinterpret_cast<f32x4*>(op + d) = f32x4{o[d] * inv, o[d + 1] * inv, o[d + 2] * inv, o[d + 3] * inv};
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *reinterpret_cast<f32x4*>(op + dt * 32 + q4 * 8 + g * 4) =
+            f32x4{acc[dt][q4 * 4] * inv, acc[dt][q4 * 4 + 1] * inv, acc[dt][q4 * 4 + 2] * inv,
+                  acc[dt][q4 * 4 + 3] * inv};
   }
 }
 
@@ -1151,6 +1277,13 @@ __global__ void att_zero_counters(int* __restrict__ ctr, int n) {
   if (i < n) ctr[i] = 0;
 }
 
+// A call's relative-position bias and key padding (AttnArgs::diag, keep).
+struct AttnBias {
+  const float* diag;
+  int64_t diag_ld;
+  const uint8_t* keep;
+  int64_t keep_ld;
+};
 // The second key segment of a joint call (seq_k2 > 0) and its per-batch count of attending keys.
 struct AttnSecond {
   const void* k;
@@ -1173,7 +1306,8 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
                           int mask_dtype, const int64_t* mask_strides, const int32_t* bound_min,
                           const int32_t* bound_max, const int64_t* bound_strides,
                           void* workspace, int64_t workspace_bytes, bool clear_counters,
-                          difflet_stream_t stream, const AttnSecond* second = nullptr) {
+                          difflet_stream_t stream, const AttnSecond* second = nullptr,
+                          const AttnBias* bias = nullptr) {
   DLT_REQUIRE(q && k && v && o && q_strides && k_strides && v_strides && o_strides,
               DIFFLET_EINVAL, "attention: null pointer");
   DLT_REQUIRE(dtype == DIFFLET_BF16 || dtype == DIFFLET_F16 || dtype == DIFFLET_F32,
@@ -1231,7 +1365,8 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   const bool masked = causal || mask || bound_min || !(scale > 0.0f);
   const bool bounded = bound_min && !causal && scale > 0.0f;
   const bool gen = second || bounded;  // the ping-pong kernel's instance for windows and segments
-  const bool pingpong = second || (head_dim == HD && (!masked || bounded) && seq_k > 1024);
+  const bool pingpong =
+      second || (head_dim == HD && (!masked || bounded) && !bias && seq_k > 1024);
   const int qblock = pingpong ? 2 * BLOCK_M : BLOCK_M;  // queries per workgroup
   args.q_tiles = (int)((seq_q + qblock - 1) / qblock);
   const int64_t total = (int64_t)args.q_tiles * batch * heads;
@@ -1247,6 +1382,13 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   args.bmax = bound_max;
   if (bound_min)
     for (int i = 0; i < 3; ++i) args.bs[i] = bound_strides[i];
+  if (bias) {
+    args.diag = bias->diag;
+    args.diag_ld = bias->diag_ld;
+    args.keep = bias->keep;
+    args.keep_ld = bias->keep_ld;
+  }
+  const int mode = bias ? 2 : masked ? 1 : 0;
   args.key_tiles = (int)((seq_k + BLOCK_N - 1) / BLOCK_N);
   args.seq_k1 = (int)seq_k;
   args.j1 = INT_MAX;
@@ -1267,19 +1409,29 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
     }
   }
   hipStream_t s = (hipStream_t)stream;
+  using D64 = std::integral_constant<int, 64>;
+  using D128 = std::integral_constant<int, 128>;
+  using M0 = std::integral_constant<int, 0>;
+  using M1 = std::integral_constant<int, 1>;
+  using M2 = std::integral_constant<int, 2>;
+  auto with_mode = [&](auto f) {
+    if (mode == 0) f(M0{});
+    else if (mode == 1) f(M1{});
+    else f(M2{});
+  };
   if (dtype == DIFFLET_F32) {
-    const int cus = att_device_cus();
-    const bool narrow = (int64_t)((seq_q + 255) / 256) * batch * heads < 2 * (cus > 0 ? cus : 256);
-    const int nq = narrow ? 64 : 256;
-    args.q_tiles = (int)((seq_q + nq - 1) / nq);
+    args.q_tiles = (int)((seq_q + BLOCK_M - 1) / BLOCK_M);
     const int64_t t32 = (int64_t)args.q_tiles * batch * heads;
     DLT_REQUIRE(t32 < (1LL << 31), DIFFLET_EUNSUPPORTED, "%s: too many tiles", name);
     args.total = (int)t32;
-    const dim3 g32((unsigned)t32);
-    if (head_dim == 64 && narrow) hipLaunchKernelGGL((attn_f32_kernel<64, 64>), g32, dim3(64), 0, s, args);
-    else if (head_dim == 64) hipLaunchKernelGGL((attn_f32_kernel<64, 256>), g32, dim3(256), 0, s, args);
-    else if (narrow) hipLaunchKernelGGL((attn_f32_kernel<128, 64>), g32, dim3(64), 0, s, args);
-    else hipLaunchKernelGGL((attn_f32_kernel<128, 256>), g32, dim3(256), 0, s, args);
+    with_mode([&](auto m) {
+      constexpr int MODE = decltype(m)::value;
+      const dim3 g32((unsigned)t32);
+      if (head_dim == 64)
+        hipLaunchKernelGGL((attn_f32_kernel<64, MODE>), g32, dim3(256), 0, s, args);
+      else
+        hipLaunchKernelGGL((attn_f32_kernel<128, MODE>), g32, dim3(256), 0, s, args);
+    });
     return dlt_check_launch(name);
   }
   dim3 grid((unsigned)total);
@@ -1302,11 +1454,11 @@ static int attention_impl(const char* name, const void* q, const void* k, const 
   auto fwd = [&](auto t, auto d) {
     using TT = decltype(t);
     constexpr int DD = decltype(d)::value;
-    if (masked) hipLaunchKernelGGL((attn_fwd_kernel<TT, true, DD>), grid, dim3(256), 0, s, args);
-    else hipLaunchKernelGGL((attn_fwd_kernel<TT, false, DD>), grid, dim3(256), 0, s, args);
+    with_mode([&](auto m) {
+      constexpr int MODE = decltype(m)::value;
+      hipLaunchKernelGGL((attn_fwd_kernel<TT, MODE, DD>), grid, dim3(256), 0, s, args);
+    });
   };
-  using D64 = std::integral_constant<int, 64>;
-  using D128 = std::integral_constant<int, 128>;
   if (dtype == DIFFLET_BF16) {
     if (pingpong && gen) hipLaunchKernelGGL((attn_pp_kernel<bf16, true>), grid, dim3(512), 0, s, args);
     else if (pingpong) hipLaunchKernelGGL((attn_pp_kernel<bf16, false>), grid, dim3(512), 0, s, args);
@@ -1371,6 +1523,25 @@ extern "C" int difflet_rocm_attention_joint(
                         q_strides, k_strides, v_strides, o_strides, scale, 0, nullptr, 0, nullptr,
                         nullptr, nullptr, nullptr, workspace, workspace_bytes, false, stream,
                         &second);
+}
+
+extern "C" int difflet_rocm_attention_relative_bias(
+    const void* q, const void* k, const void* v, void* o, int dtype, int64_t batch, int64_t heads,
+    int64_t seq_q, int64_t seq_k, int64_t head_dim, const int64_t* q_strides,
+    const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides, float scale,
+    const float* diag, int64_t diag_stride, const uint8_t* key_keep, int64_t keep_stride,
+    difflet_stream_t stream) {
+  DLT_REQUIRE(diag && ((uintptr_t)diag & 3) == 0, DIFFLET_EINVAL,
+              "attention_relative_bias: diag missing");
+  DLT_REQUIRE(diag_stride >= seq_q + seq_k + 2 && diag_stride < (1LL << 30), DIFFLET_EINVAL,
+              "attention_relative_bias: diag rows hold seq_q + seq_k - 1 values and 3 of padding");
+  DLT_REQUIRE(!key_keep || keep_stride >= seq_k, DIFFLET_EINVAL,
+              "attention_relative_bias: keep_stride shorter than seq_k");
+  const AttnBias bias = {diag, diag_stride, key_keep, keep_stride};
+  return attention_impl("attention_relative_bias", q, k, v, o, dtype, batch, heads, seq_q, seq_k,
+                        head_dim, q_strides, k_strides, v_strides, o_strides, scale, 0, nullptr, 0,
+                        nullptr, nullptr, nullptr, nullptr, nullptr, 0, false, stream, nullptr,
+                        &bias);
 }
 
 // ---- attention that allocates nothing: the split schedule's workspace is this file's static

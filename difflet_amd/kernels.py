@@ -151,6 +151,37 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float
     return out
 
 
+def attention_relative_bias(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float,
+                            diag: torch.Tensor, key_keep: torch.Tensor | None = None,
+                            out: torch.Tensor | None = None) -> torch.Tensor:
+    """softmax(q k^T scale + diag[h, k - q + Sq - 1]) v on [B, H, S, D] tensors; keys with
+    key_keep[b, k] == 0 (bool / uint8 [B, Sk]) are masked. diag: contiguous fp32 [H, Sq + Sk + 2],
+    the last 3 columns unused."""
+    dev = _on_gpu(q, k, v, diag, key_keep, out)
+    b, h, sq, d = q.shape
+    sk = k.shape[2]
+    if not (q.dtype == k.dtype == v.dtype):
+        raise TypeError(f"q, k, v dtypes differ: {q.dtype}, {k.dtype}, {v.dtype}")
+    if k.shape != (b, h, sk, d) or v.shape != (b, h, sk, d):
+        raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
+    if diag.dtype != torch.float32 or diag.shape != (h, sq + sk + 2) or not diag.is_contiguous():
+        raise ValueError(f"diag must be a contiguous fp32 [{h}, {sq + sk + 2}]")
+    if key_keep is not None:
+        if key_keep.shape != (b, sk) or key_keep.dtype not in (torch.bool, torch.uint8):
+            raise ValueError(f"key_keep must be bool/uint8 [{b}, {sk}]")
+        key_keep = key_keep.contiguous()
+    q, k, v = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
+    if out is None:
+        out = torch.empty((b, h, sq, d), dtype=v.dtype, device=dev)
+    elif out.shape != (b, h, sq, d) or out.dtype != v.dtype or out.stride(-1) != 1:
+        raise ValueError(f"out must be {v.dtype} [{b}, {h}, {sq}, {d}] with contiguous rows")
+    check(lib().difflet_rocm_attention_relative_bias(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(out), _dt(q), b, h, sq, sk, d,
+        *(_arr(t.stride()[:3]) for t in (q, k, v, out)), float(scale), _ptr(diag), diag.shape[1],
+        _ptr(key_keep), sk, _stream(dev)), "attention_relative_bias")
+    return out
+
+
 def attention_joint(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k2: torch.Tensor,
                     v2: torch.Tensor, *, scale: float, key_count: torch.Tensor | None = None,
                     count_offset: int = 0) -> torch.Tensor:

@@ -175,6 +175,7 @@ class T5Encoder:
         # the residual epilogue of the bf16 GEMM is residual + gate * (x W^T): a gate of ones
         self._ones = torch.ones(1, cfg.d_model, dtype=torch.bfloat16, device=self.device)
         self._buckets: dict[int, torch.Tensor] = {}
+        self._diag_buckets: dict[int, torch.Tensor] = {}
 
     # ------------------------------------------------------------------ pieces
     def buckets(self, s: int) -> torch.Tensor:
@@ -184,6 +185,14 @@ class T5Encoder:
                                           self.cfg.relative_attention_max_distance).to(self.device)
             self._buckets[s] = b
         return b
+
+    def _bias_diag(self, table, s: int) -> torch.Tensor:
+        """The position bias of a head depends on key minus query alone: fp32 [H, 2 s + 2], entry j
+        for the difference j - (s - 1) (the last 3 pad the attention kernel's 16-byte reads)."""
+        b = self._diag_buckets.get(s)
+        if b is None:
+            b = self._diag_buckets[s] = torch.nn.functional.pad(self.buckets(s), (0, 3))
+        return kernels.relative_bias(b, table, batch=1, seq_q=1, seq_k=2 * s + 2).view(-1, 2 * s + 2)
 
     def _linear(self, x, w, out, residual=None):
         if self.dtype == torch.float32:
@@ -197,13 +206,14 @@ class T5Encoder:
             epi = _lib.EPI_GATE_RESIDUAL
         kernels.gemm_grouped([p], kind="bf16", epilogue=epi, workspace="shared")
 
-    def _attention(self, qkv, att, bias, b, s):
+    def _attention(self, qkv, att, diag, keep, b, s):
         cfg = self.cfg
         h, dk, inner = cfg.num_heads, cfg.d_kv, cfg.inner_dim
         view = lambda t, off, ld: t.as_strided((b, h, s, dk), (s * ld, dk, ld, 1),  # noqa: E731
                                                t.storage_offset() + off)
         q, k, v = (view(qkv, i * inner, 3 * inner) for i in range(3))
-        kernels.attention(q, k, v, scale=1.0, attention_mask=bias, out=view(att, 0, inner))
+        kernels.attention_relative_bias(q, k, v, scale=1.0, diag=diag, key_keep=keep,
+                                        out=view(att, 0, inner))
 
     # ------------------------------------------------------------------ forward
     def forward(self, input_ids: torch.Tensor,
@@ -229,15 +239,14 @@ class T5Encoder:
         att = torch.empty(rows, cfg.inner_dim, dtype=dt, device=dev)
         ff = torch.empty(rows, 2 * cfg.d_ff, dtype=dt, device=dev)
         g = torch.empty(rows, cfg.d_ff, dtype=dt, device=dev)
-        bias = None
+        diag = None
         eps = cfg.layer_norm_epsilon
         for lay in self.layers:
             if "rel" in lay:
-                bias = kernels.relative_bias(self.buckets(s), lay["rel"], batch=b if keep is not None else 1,
-                                             seq_q=s, seq_k=s, key_keep=keep)
+                diag = self._bias_diag(lay["rel"], s)
             n = kernels.rms_norm(x, lay["ln0"], eps)
             self._linear(n, lay["wqkv"], qkv)
-            self._attention(qkv, att, bias, b, s)
+            self._attention(qkv, att, diag, keep, b, s)
             self._linear(att, lay["wo_attn"], x, residual=x)
             n = kernels.rms_norm(x, lay["ln1"], eps)
             self._linear(n, lay["wi"], ff)

@@ -54,8 +54,7 @@ int difflet_rocm_device_count(void);
  * semantics are the CPU oracle's, difflet/backends/cpu/ops_impl/attention.py:8-48:
  *   out = softmax(q k^T * scale [+ mask]) v, softmax in fp32, output in v's dtype.
  * q: [batch, heads, seq_q, head_dim] addressed by strides {b, h, s}; k, v: [.., seq_k, ..];
- * o: like q. head_dim 64 or 128; dtype BF16 or F16 (matrix-core kernels) or F32 (a VALU
- * kernel, one query per lane).
+ * o: like q. head_dim 64 or 128; dtype BF16, F16 or F32 (the fp32 matrix cores: fp32 throughout).
  * causal: key j > query i is masked. mask: optional, [batch, heads, seq_q, seq_k] through
  * strides (0 broadcasts); BOOL (nonzero attends) or F32/BF16/F16 additive. bound_min /
  * bound_max: optional int32 [batch, heads, seq_q] through strides; keys in [min, max) attend
@@ -94,6 +93,21 @@ int difflet_rocm_attention_joint(const void* q, const void* k, const void* v, co
                                  const int64_t* v2_strides, const int64_t* o_strides, float scale,
                                  const int32_t* key_count, int64_t count_offset, void* workspace,
                                  int64_t workspace_bytes, difflet_stream_t stream);
+
+/* Attention with a relative-position bias, as the T5 encoders compute it
+ * (difflet/models/flux/modeling_t5.py:200-248): difflet_rocm_attention with the additive fp32 mask
+ * diag[h][k - q + seq_q - 1] and, where key_keep is given, keys with key_keep[b][k] == 0 masked,
+ * without the [batch, heads, seq_q, seq_k] table. diag: fp32 [heads], rows of diag_stride >=
+ * seq_q + seq_k + 2 floats (seq_q + seq_k - 1 used). key_keep: optional bytes [batch], rows of
+ * keep_stride. All dtypes and head dims of difflet_rocm_attention. */
+int difflet_rocm_attention_relative_bias(const void* q, const void* k, const void* v, void* o,
+                                         int dtype, int64_t batch, int64_t heads, int64_t seq_q,
+                                         int64_t seq_k, int64_t head_dim,
+                                         const int64_t* q_strides, const int64_t* k_strides,
+                                         const int64_t* v_strides, const int64_t* o_strides,
+                                         float scale, const float* diag, int64_t diag_stride,
+                                         const uint8_t* key_keep, int64_t keep_stride,
+                                         difflet_stream_t stream);
 
 /* Bytes of attention workspace the split schedule needs on the current device: 16 KiB of
  * counters + 2 x 132 KiB per compute unit (0 without a device). No counterpart in the

@@ -100,3 +100,30 @@ def test_bounded_attention_per_query_windows(gpu, dtype, scale):
     out = A.attention(q.to(gpu), k.to(gpu), v.to(gpu), scale=scale, bound_min=lo.to(gpu),
                       bound_max=hi.to(gpu))
     assert rel_l2(out, ref) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk,padded", [(1, 1, False), (33, 64, True), (128, 65, True),
+                                          (129, 200, False), (226, 226, True)])
+def test_relative_bias_attention(gpu, dtype, d, sq, sk, padded):
+    """The relative-position bias read by its diagonals, with key padding (a batch element whose
+    keys are all padding averages v), against the expanded additive mask. fp32: sums of d and sk
+    terms in fp32, rel L2 < 1e-5."""
+    from difflet_amd import kernels
+
+    print(f"relative bias {dtype} {d} {sq} {sk} {padded}", flush=True)
+    g = torch.Generator().manual_seed(sq + sk)
+    q, k, v = (torch.randn(2, 3, s, d, generator=g).to(dtype) for s in (sq, sk, sk))
+    diag = torch.randn(3, sq + sk + 2, generator=g)
+    j = torch.arange(sk)[None, :] - torch.arange(sq)[:, None] + sq - 1
+    bias, keep = diag[:, j][None].expand(2, -1, -1, -1), None
+    if padded:
+        keep = torch.rand(2, sk, generator=g) > 0.4
+        keep[1] = False
+        bias = bias.masked_fill(~keep[:, None, None, :], torch.finfo(torch.float32).min)
+    ref = ops.attention(q.float(), k.float(), v.float(), scale=0.3, attention_mask=bias)
+    out = kernels.attention_relative_bias(q.to(gpu), k.to(gpu), v.to(gpu), scale=0.3,
+                                          diag=diag.to(gpu),
+                                          key_keep=None if keep is None else keep.to(gpu))
+    assert rel_l2(out, ref) < TOL.get(dtype, 1e-5)
