@@ -98,7 +98,8 @@ def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) 
         x = F.pad(x, (0, k_pad - kx))
     if bias is not None and bias.shape[0] != n_pad:
         bias = F.pad(bias, (0, n_pad - bias.shape[0]))
-    y = kernels.gemm_f32(x.contiguous(), w, None if bias is None else bias.contiguous())
+    y = kernels.gemm_f32(x.contiguous(), w, None if bias is None else bias.contiguous(),
+                         workspace="call")
     return y if n_pad == out_features else y[:, :out_features].contiguous()
 
 

@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_kernel(const GemmArgs args) 
 }
 
 // Compute units of the current device (one GEMM workgroup fits a CU: its LDS use is > 80 KB).
-static int device_cus() {
+int gemm_device_cus() {
   static int cached[64] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
@@ -1066,7 +1066,7 @@ template <Elem E> constexpr SmallElem small_elem() {
 // (measured within 10 % at 24 to 288 tiles).
 template <Elem E>
 static SmallPlan small_plan_of(int64_t m, int64_t n, int64_t k, int64_t scratch, const SkPlan& sk) {
-  const int cus = device_cus();
+  const int cus = gemm_device_cus();
   if (cus <= 0) return SmallPlan{0, 0, 0, 0};
   const int64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
   const int nk = (int)(k / ElemTraits<E>::KT);
@@ -1221,7 +1221,7 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
     args.rope_sin = qk->sin;
   }
   args.sk = sk_plan((int)tiles, (int)(k / KT), E == Elem::MX ? 4 : 1,
-                    workspace ? device_cus() : 0, workspace ? workspace_bytes : 0);
+                    workspace ? gemm_device_cus() : 0, workspace ? workspace_bytes : 0);
   // launches of few tiles: smaller tiles, K cut into pieces (gemm_small.hip)
   if (nproblems == 1 && !qk &&
       (epilogue == DIFFLET_EPI_NONE || epilogue == DIFFLET_EPI_GATE_RESIDUAL)) {
@@ -1281,7 +1281,7 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
 using namespace dlt;
 
 extern "C" int64_t difflet_rocm_gemm_workspace_bytes(void) {
-  const int cus = device_cus();
+  const int cus = gemm_device_cus();
   return cus > 0 ? sk_workspace_bytes(cus) : 0;
 }
 
@@ -1292,7 +1292,8 @@ extern "C" int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t 
   const SkPlan whole = {};
   const SmallPlan p = kind == 0   ? small_plan_of<Elem::BF16>(m, n, k, cap, whole)
                       : kind == 1 ? small_plan_of<Elem::FP8>(m, n, k, cap, whole)
-                                  : small_plan_of<Elem::MX>(m, n, k, cap, whole);
+                      : kind == 2 ? small_plan_of<Elem::MX>(m, n, k, cap, whole)
+                                  : small_plan(SmallElem::F32, m, n, k, gemm_device_cus(), cap, 2e30);
   return p.pieces > 1 ? SK_CTR_BYTES + p.pieces * m * n * 4 : 0;
 }
 

@@ -8,8 +8,10 @@
 // the stage's 32 indices onto the 16 MFMA steps x 2 halves), so each lane reads its 16 values
 // of a row with four 16-byte LDS reads.
 //
-// The same kernel runs the fp32 causal convolutions of the VAE decoders as implicit GEMMs: the A
-// loader gathers each row's 4-float runs from the frames (difflet_rocm_conv_causal).
+// This file's kernel runs the fp32 causal convolutions of the VAE decoders as implicit GEMMs: the A
+// loader gathers each row's 4-float runs from the frames (difflet_rocm_conv_causal). Plain GEMMs
+// run in gemm_small.hip, with the same K order and so the same sums, unless a row is longer than
+// its 32-bit offsets reach.
 //
 // Workgroup tile 64 (M) x 128 (N), 4 waves of 32 x 64 (two 32 x 32 MFMA tiles); A and W stages
 // of 32 floats per row in LDS, double-buffered (55 KB: two workgroups per compute unit), the
@@ -24,6 +26,7 @@
 
 #include "common.hpp"
 #include "difflet_rocm.h"
+#include "gemm_small.hpp"
 
 namespace dlt {
 
@@ -187,10 +190,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmF32Args p) {
 
 using namespace dlt;
 
-extern "C" int difflet_rocm_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw,
-                                     const float* bias, const float* residual, int64_t ldr,
-                                     float* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
-                                     difflet_stream_t stream) {
+extern "C" int difflet_rocm_gemm_f32_scratch(const float* a, int64_t lda, const float* w,
+                                             int64_t ldw, const float* bias, const float* residual,
+                                             int64_t ldr, float* c, int64_t ldc, int64_t m,
+                                             int64_t n, int64_t k, void* scratch,
+                                             int64_t scratch_bytes, difflet_stream_t stream) {
   DLT_REQUIRE(m >= 0 && n > 0 && k > 0, DIFFLET_EINVAL,
               "gemm_f32: need m >= 0 and positive n, k (m=%lld n=%lld k=%lld)", (long long)m,
               (long long)n, (long long)k);
@@ -209,6 +213,29 @@ extern "C" int difflet_rocm_gemm_f32(const float* a, int64_t lda, const float* w
                 "gemm_f32: pointers must be 16-byte aligned");
   const int64_t tiles_m = (m + F32_BM - 1) / F32_BM, tiles_n = (n + F32_BN - 1) / F32_BN;
   DLT_REQUIRE(tiles_m * tiles_n < (1LL << 31), DIFFLET_EUNSUPPORTED, "gemm_f32: too many tiles");
+  DLT_REQUIRE(!scratch || ((uintptr_t)scratch & 15) == 0, DIFFLET_EINVAL,
+              "gemm_f32: scratch must be 16-byte aligned");
+  // the kernel addresses 256 rows of an operand in 32 bits; longer rows keep this file's kernel
+  constexpr int64_t kMaxLd = 1LL << 22, kMaxDim = 1LL << 30;
+  if (lda < kMaxLd && ldw < kMaxLd && m < kMaxDim && n < kMaxDim) {
+    const SmallPlan plan = small_plan(SmallElem::F32, m, n, k, gemm_device_cus(),
+                                      scratch ? scratch_bytes : 0, 2e30);
+    if (plan.bm > 0) {
+      difflet_gemm_problem q{};
+      q.a = a;
+      q.lda = lda;
+      q.w = w;
+      q.ldw = ldw;
+      q.c = c;
+      q.ldc = ldc;
+      q.bias = bias;
+      q.residual = residual;
+      q.ldr = ldr;
+      q.m = m;
+      gemm_small(SmallElem::F32, plan, q, n, k, false, m, scratch, (hipStream_t)stream);
+      return dlt_check_launch("gemm_f32");
+    }
+  }
   GemmF32Args args{};
   args.a = a;
   args.w = w;
@@ -228,6 +255,14 @@ extern "C" int difflet_rocm_gemm_f32(const float* a, int64_t lda, const float* w
   hipLaunchKernelGGL((gemm_f32_kernel<false>), dim3((unsigned)args.tiles), dim3(256), 0,
                      (hipStream_t)stream, args);
   return dlt_check_launch("gemm_f32");
+}
+
+extern "C" int difflet_rocm_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw,
+                                     const float* bias, const float* residual, int64_t ldr,
+                                     float* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
+                                     difflet_stream_t stream) {
+  return difflet_rocm_gemm_f32_scratch(a, lda, w, ldw, bias, residual, ldr, c, ldc, m, n, k,
+                                       nullptr, 0, stream);
 }
 
 namespace dlt {

@@ -17,6 +17,13 @@
 // wave has waited for its own loads of the next stage (the younger ones stay in flight), so the
 // barrier publishes that stage and frees this one's slot for the loads of stage kt + NSLOT.
 //
+// fp32 operands run here at every size (v_mfma_f32_32x32x2_f32, a stage of 32 floats per row,
+// lane half h of a fragment taking floats 16 h .. 16 h + 15 in turn): each stage is 4096 cycles of
+// MFMA per SIMD for 32 KB, so the matrix cores are the bound, and the ring with one barrier per
+// stage and fragments read a step ahead keeps them fed where the register-staged kernel
+// (gemm_f32.hip, which the convolutions still use, with the same K order and so the same bits)
+// reached two thirds of their rate: UMT5's four linears of 452 rows 1936 -> F32SUM us.
+//
 // K pieces: piece c of a tile writes its fp32 sums to part[c][m][n]; gemm_small_reduce adds the
 // pieces in order and runs the epilogue. Nothing is kept between launches and nobody waits, so
 // any scratch buffer serves, on any stream and under graph capture.
@@ -31,9 +38,9 @@ struct SmallArgs {
   const uint8_t* a;
   const uint8_t* w;
   uint8_t* c;
-  const bf16* bias;
-  const bf16* gate;
-  const bf16* res;
+  const void* bias;  // bf16 (F32: fp32), as gate, res and C
+  const void* gate;
+  const void* res;
   const uint8_t* a_scale;
   const uint8_t* w_scale;
   int64_t lda, ldw, ldc, ldr, gate_stride, rows_per_batch;  // element strides
@@ -71,6 +78,28 @@ template <SmallElem E, bool GATE>
 __device__ __forceinline__ void small_store8(const SmallArgs& a, int64_t m, int64_t n, float* v) {
   if (n >= a.n) return;
   const bool full = n + 8 <= a.n;  // n % 4 == 0: a chunk is full or half full
+  if constexpr (E == SmallElem::F32) {
+    const float* bias = reinterpret_cast<const float*>(a.bias);
+    const float* res = reinterpret_cast<const float*>(a.res);
+    float* dst = reinterpret_cast<float*>(a.c) + m * a.ldc + n;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h == 1 && !full) break;
+      f32x4 x = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+      if (bias) {
+        const f32x4 b = *reinterpret_cast<const f32x4*>(bias + n + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] += b[e];
+      }
+      if (res) {
+        const f32x4 r = *reinterpret_cast<const f32x4*>(res + m * a.ldr + n + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = r[e] + x[e];
+      }
+      *reinterpret_cast<f32x4*>(dst + 4 * h) = x;
+    }
+    return;
+  }
   auto load8 = [&](const bf16* p, float* o) {
     const u32x2 lo = *reinterpret_cast<const u32x2*>(p);
     const u32x2 hi = full ? *reinterpret_cast<const u32x2*>(p + 4) : u32x2{0u, 0u};
@@ -90,14 +119,14 @@ __device__ __forceinline__ void small_store8(const SmallArgs& a, int64_t m, int6
   }
   if (a.bias) {
     float b[8];
-    load8(a.bias + n, b);
+    load8(reinterpret_cast<const bf16*>(a.bias) + n, b);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] += b[e];
   }
   if constexpr (GATE) {
     float g[8], r[8];
-    load8(a.gate + m / a.rows_per_batch * a.gate_stride + n, g);
-    load8(a.res + m * a.ldr + n, r);
+    load8(reinterpret_cast<const bf16*>(a.gate) + m / a.rows_per_batch * a.gate_stride + n, g);
+    load8(reinterpret_cast<const bf16*>(a.res) + m * a.ldr + n, r);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = r[e] + g[e] * v[e];
   }
@@ -115,12 +144,13 @@ __device__ __forceinline__ void small_store8(const SmallArgs& a, int64_t m, int6
 
 template <SmallElem E, int BM, int BN, int NSLOT, bool GATE>
 __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args) {
-  constexpr int EB = E == SmallElem::BF16 ? 2 : 1;
+  constexpr bool F32 = E == SmallElem::F32;
+  constexpr int EB = F32 ? 4 : E == SmallElem::BF16 ? 2 : 1;
   constexpr int WAVES_M = BM == 256 ? 4 : 2, WAVES_N = 8 / WAVES_M;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int TI = WTM / 32, TJ = WTN / 32;     // MFMA tiles per wave
-  constexpr int NKS = E == SmallElem::BF16 ? 4 : 2;  // MFMA K steps per stage
-  constexpr int NA = E == SmallElem::BF16 ? 1 : 2;   // 16-byte LDS reads per fragment
+  constexpr int NKS = EB > 1 ? 4 : 2;  // K steps per stage (F32: of 4 MFMAs each)
+  constexpr int NA = EB > 1 ? 1 : 2;   // 16-byte LDS reads per fragment
   constexpr int SA = BM / 64, SW = BN / 64, LPS = SA + SW;  // 1 KB loads per wave and stage
   constexpr int SLOT = (BM + BN) * 128;
   // MX: E8M0 scales of 4 stages (16 bytes) per row, a ring of two such blocks
@@ -147,7 +177,7 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
   const int tn = rest % args.tiles_n, piece = rest / args.tiles_n;
   const int m0 = tm * BM, n0 = tn * BN;
   const int M = args.m, N = args.n;
-  const int nk = args.k / (128 / EB);
+  const int nk = (args.k + 128 / EB - 1) / (128 / EB);  // F32: the last stage may be partial
   const int kbeg = piece * args.piece_stages;
   const int nkt = min(args.piece_stages, nk - kbeg);
 
@@ -191,11 +221,21 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
     const uint32_t kb = kt < nkt ? (uint32_t)(kbeg + kt) * 128u : 0u;
     const uint32_t off = kt < nkt ? 0u : 0x80000000u;
     uint8_t* d = lds + st * SLOT;
+    // F32: K is a multiple of 4, so a lane's 16 bytes are all inside K or all past it
+    auto at = [&](uint32_t o, int slab) {
+      if constexpr (F32) {
+        const int r = slab * 8 + (lane >> 3);
+        const int kk = (kbeg + kt) * 32 + ((lane & 7) ^ swz8s(r)) * 4;
+        return kt < nkt && kk < args.k ? o : 0xfffffff0u;
+      }
+      return o | off;
+    };
 #pragma unroll
-    for (int i = 0; i < SA; ++i) dma16s(ra, d + (wave * SA + i) * 1024, aoff[i] | off, kb);
+    for (int i = 0; i < SA; ++i)
+      dma16s(ra, d + (wave * SA + i) * 1024, at(aoff[i], wave * SA + i), kb);
 #pragma unroll
     for (int i = 0; i < SW; ++i)
-      dma16s(rw, d + BM * 128 + (wave * SW + i) * 1024, woff[i] | off, kb);
+      dma16s(rw, d + BM * 128 + (wave * SW + i) * 1024, at(woff[i], wave * SW + i), kb);
   };
 
   f32x16 acc[4][4];  // [i < TI][j < TJ]
@@ -209,7 +249,7 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
   auto read_frags = [&](const uint8_t* stage, int ks, int set) {
 #pragma unroll
     for (int h = 0; h < NA; ++h) {
-      const int ch = 2 * NA * ks + 2 * h + fhalf;
+      const int ch = F32 ? 4 * fhalf + ks : 2 * NA * ks + 2 * h + fhalf;
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
         const int r = wn * WTN + j * 32 + frow;
@@ -248,7 +288,12 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
       for (int j = 0; j < TJ; ++j) {
         const i32x4* w = fw[set][j];
         const i32x4* x = fa[set][i];
-        if constexpr (E == SmallElem::BF16) {
+        if constexpr (F32) {
+          const f32x4 wv = __builtin_bit_cast(f32x4, w[0]), xv = __builtin_bit_cast(f32x4, x[0]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[e], xv[e], acc[i][j], 0, 0, 0);
+        } else if constexpr (E == SmallElem::BF16) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[0]),
                                                               __builtin_bit_cast(bf16x8, x[0]),
                                                               acc[i][j], 0, 0, 0);
@@ -375,8 +420,8 @@ __global__ __launch_bounds__(256) void gemm_small_reduce(const SmallArgs args) {
 }
 
 // Estimated times on MI355X, in us, from sweeps over 16 to 3000 rows of the layers' widths:
-//  - a workgroup takes kStage per K stage (64-, 128- and 256-row tiles; the MX scales cost the
-//    small tiles LDS reads) plus 5 for its first loads and its output; a launch runs
+//  - a workgroup takes kStage per K stage (bf16, fp8, MXFP8, fp32; 64-, 128- and 256-row tiles;
+//    the MX scales cost the small tiles LDS reads, fp32 is the MFMAs' time) plus 5 for its first loads and its output; a launch runs
 //    ceil(workgroups / units) rounds of that, but no faster than its weights come from HBM;
 //  - cutting K adds the reduce launch and the sums' trip out and back at about 5 TB/s.
 // 16 and 8 rows apart from the boundary the choices measured (bf16, K = N = 3072 / 12288 x 3072 /
@@ -387,21 +432,24 @@ __global__ __launch_bounds__(256) void gemm_small_reduce(const SmallArgs args) {
 SmallPlan small_plan(SmallElem e, int64_t m, int64_t n, int64_t k, int cus, int64_t scratch,
                      double big_us) {
   SmallPlan best = {0, 0, 0, 0};
-  if (cus <= 0 || m <= 0 || m > 4096) return best;
-  const int eb = e == SmallElem::BF16 ? 2 : 1;
-  const int nk = (int)(k * eb / 128), gran = e == SmallElem::MX ? 4 : 1;
+  const bool f32 = e == SmallElem::F32;
+  if (cus <= 0 || m <= 0 || (m > 4096 && !f32)) return best;
+  const int eb = f32 ? 4 : e == SmallElem::BF16 ? 2 : 1;
+  const int nk = (int)((k * eb + 127) / 128), gran = e == SmallElem::MX ? 4 : 1;
   // PLAN
   static const int kRows[3] = {64, 128, 256};
-  static const double kStage[3][3] = {{0.36, 0.52, 0.90}, {0.30, 0.43, 0.88}, {0.38, 0.60, 0.90}};
+  static const double kStage[4][3] = {
+      {0.36, 0.52, 0.90}, {0.30, 0.43, 0.88}, {0.38, 0.60, 0.90}, {0.90, 1.78, 3.55}};
   const double hbm_us = (double)n * k * eb / 4.5e6;
   double best_us = 0.95 * big_us;  // within the estimates' error of each other: leave it
   for (int i = 0; i < 3; ++i) {
     const int64_t tiles = ((m + kRows[i] - 1) / kRows[i]) * ((n + 127) / 128);
-    if (tiles > 4 * cus) continue;
+    if (tiles > 4 * cus && !f32) continue;
     for (int pieces = 1; pieces <= 16; ++pieces) {
       const int ps = ((nk + pieces - 1) / pieces + gran - 1) / gran * gran;
       if ((nk + ps - 1) / ps != pieces) continue;  // rounding left a piece without stages
       if (pieces > 1 && (ps < 4 || pieces * m * n * 4 > scratch)) continue;
+      if (pieces > 1 && tiles * pieces > 4 * cus) break;
       const double rounds = (double)((tiles * pieces + cus - 1) / cus);
       double us = std::max(rounds * (ps * kStage[(int)e][i] + 5.0), hbm_us);
       if (pieces > 1) us += 3.0 + (double)pieces * m * n * 8 / 5e6;
@@ -436,9 +484,9 @@ void gemm_small(SmallElem e, const SmallPlan& plan, const difflet_gemm_problem& 
   a.a = (const uint8_t*)q.a;
   a.w = (const uint8_t*)q.w;
   a.c = (uint8_t*)q.c;
-  a.bias = (const bf16*)q.bias;
-  a.gate = (const bf16*)q.gate;
-  a.res = (const bf16*)q.residual;
+  a.bias = q.bias;
+  a.gate = q.gate;
+  a.res = q.residual;
   a.a_scale = (const uint8_t*)q.a_scale;
   a.w_scale = (const uint8_t*)q.w_scale;
   a.lda = q.lda;
@@ -455,6 +503,10 @@ void gemm_small(SmallElem e, const SmallPlan& plan, const difflet_gemm_problem& 
   a.pieces = plan.pieces;
   a.piece_stages = plan.piece_stages;
   a.part = (float*)scratch;
+  if (e == SmallElem::F32) {
+    launch_small<SmallElem::F32, false>(a, plan, s);
+    return;
+  }
   auto go = [&](auto et) {
     constexpr SmallElem E = decltype(et)::value;
     if (gate) launch_small<E, true>(a, plan, s);

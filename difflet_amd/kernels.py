@@ -253,7 +253,7 @@ class QkNormRope:
 
 _GEMM_FN = {"bf16": "difflet_rocm_gemm_bf16", "fp8": "difflet_rocm_gemm_fp8_rowwise",
             "mx": "difflet_rocm_gemm_mxfp8"}
-_KIND_ID = {"bf16": 0, "fp8": 1, "mx": 2}
+_KIND_ID = {"bf16": 0, "fp8": 1, "mx": 2, "f32": 3}
 
 
 _WORKSPACE: dict[tuple[int, int], torch.Tensor] = {}
@@ -783,10 +783,11 @@ def gemm_bf16_f32out(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
-             residual: torch.Tensor | None = None, out: torch.Tensor | None = None
-             ) -> torch.Tensor:
+             residual: torch.Tensor | None = None, out: torch.Tensor | None = None,
+             workspace: str | None = None) -> torch.Tensor:
     """A W^T (+ bias) (+ residual) in fp32 on the matrix cores: a [M, K], w [N, K], bias [N],
-    residual and out [M, N] (residual may be out). K and N multiples of 4."""
+    residual and out [M, N] (residual may be out). K and N multiples of 4. workspace: None (K
+    whole, one order of sums for every M and N) or "call" (as gemm_grouped's)."""
     for name, t in (("a", a), ("w", w), ("bias", bias), ("residual", residual), ("out", out)):
         if t is not None and t.dtype != torch.float32:
             raise TypeError(f"gemm_f32: {name} must be fp32, got {t.dtype}")
@@ -805,10 +806,16 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
     a2 = a if a.stride(1) == 1 and a.stride(0) % 4 == 0 else a.contiguous()
     w2 = w if w.stride(1) == 1 and w.stride(0) % 4 == 0 else w.contiguous()
     y = out if out is not None else torch.empty((m, n), dtype=torch.float32, device=dev)
-    check(lib().difflet_rocm_gemm_f32(_ptr(a2), a2.stride(0), _ptr(w2), w2.stride(0), _ptr(bias),
-                                      _ptr(residual),
-                                      residual.stride(0) if residual is not None else 0,
-                                      _ptr(y), y.stride(0), m, n, k, _stream(dev)), "gemm_f32")
+    scratch = None
+    if workspace == "call":
+        nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID["f32"], m, n, k)
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    elif workspace is not None:
+        raise ValueError(f"workspace must be 'call' or None, got {workspace!r}")
+    check(lib().difflet_rocm_gemm_f32_scratch(
+        _ptr(a2), a2.stride(0), _ptr(w2), w2.stride(0), _ptr(bias), _ptr(residual),
+        residual.stride(0) if residual is not None else 0, _ptr(y), y.stride(0), m, n, k,
+        _ptr(scratch), 0 if scratch is None else scratch.numel(), _stream(dev)), "gemm_f32")
     return y
 
 

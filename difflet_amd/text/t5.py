@@ -196,7 +196,7 @@ class T5Encoder:
 
     def _linear(self, x, w, out, residual=None):
         if self.dtype == torch.float32:
-            kernels.gemm_f32(x, w, residual=residual, out=out)
+            kernels.gemm_f32(x, w, residual=residual, out=out, workspace="call")
             return
         if residual is None:
             p = kernels.Problem(x, w, out)

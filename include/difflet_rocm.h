@@ -235,8 +235,8 @@ typedef struct difflet_gemm_qk {
  * (torch.nn.functional.linear, difflet/backends/cpu/ops_impl/linear.py:9-41). */
 int64_t difflet_rocm_gemm_workspace_bytes(void);
 
-/* Bytes of scratch with which one m x n x k problem (kind 0 bf16, 1 fp8 per row, 2 MXFP8; epilogue
- * NONE or GATE_RESIDUAL) runs at its fastest among the small-launch plans: passed as the
+/* Bytes of scratch with which one m x n x k problem (kind 0 bf16, 1 fp8 per row, 2 MXFP8, 3
+ * fp32; epilogue NONE or GATE_RESIDUAL) runs at its fastest among the small-launch plans: passed as the
  * workspace, not zeroed, used by that launch only. 0: no scratch helps. Always less than
  * difflet_rocm_gemm_workspace_bytes, so such a buffer never serves the split schedule, which
  * needs zeroed counters. */
@@ -430,6 +430,14 @@ int difflet_rocm_timestep_embedding(const float* t, void* y, int dtype, int64_t 
 int difflet_rocm_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw,
                           const float* bias, const float* residual, int64_t ldr, float* c,
                           int64_t ldc, int64_t m, int64_t n, int64_t k, difflet_stream_t stream);
+
+/* difflet_rocm_gemm_f32 with scratch of difflet_rocm_gemm_scratch_bytes(3, m, n, k) bytes (16-byte
+ * aligned, not zeroed, this launch's own): launches of few tiles may then cut K into pieces, whose
+ * sums a second kernel adds in order. NULL: K stays whole. */
+int difflet_rocm_gemm_f32_scratch(const float* a, int64_t lda, const float* w, int64_t ldw,
+                                  const float* bias, const float* residual, int64_t ldr, float* c,
+                                  int64_t ldc, int64_t m, int64_t n, int64_t k, void* scratch,
+                                  int64_t scratch_bytes, difflet_stream_t stream);
 
 /* y[r, c] = gelu_tanh(x[r, c]) * x[r, f + c] for c < f: the gated FFN's act(wi_0(h)) * wi_1(h)
  * with gelu_new (difflet/models/flux/t5/modeling_t5.py:133-136,

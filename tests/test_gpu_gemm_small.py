@@ -70,3 +70,25 @@ def test_small_gemm_in_a_replayed_graph(gpu):
         torch.cuda.synchronize()
         assert torch.equal(y, eager)
     assert not torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4, 4), (63, 124, 36), (64, 128, 64), (65, 132, 100),
+                                   (16, 12288, 4096), (129, 260, 4092), (452, 4096, 1024),
+                                   (300, 512, 10240), (4200, 384, 516)])
+def test_fp32_gemm(gpu, m, n, k):
+    """fp32 GEMM: partial K stages, strided operands, residual in place; K whole and cut. Sums of k
+    products in fp32 against 64 bits: error of the sum below sqrt(k) 2^-24 relative, 1e-5 at most."""
+    print(f"fp32 gemm m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k + 8, generator=g)[:, 4:k + 4]
+    w = torch.randn(n, k + 4, generator=g)[:, :k]
+    b, r = torch.randn(n, generator=g), torch.randn(m, n, generator=g)
+    ref = a.double() @ w.double().t() + b.double()
+    ag, wg = torch.zeros(m, k + 8).to(gpu)[:, 4:k + 4], torch.zeros(n, k + 4).to(gpu)[:, :k]
+    ag.copy_(a), wg.copy_(w)
+    for workspace in (None, "call"):
+        y = kernels.gemm_f32(ag, wg, b.to(gpu), workspace=workspace)
+        assert ((y.double().cpu() - ref).norm() / ref.norm()).item() < 1e-5
+        y = r.to(gpu)
+        kernels.gemm_f32(ag, wg, b.to(gpu), residual=y, out=y, workspace=workspace)
+        assert ((y.double().cpu() - ref - r.double()).norm() / ref.norm()).item() < 1e-5
