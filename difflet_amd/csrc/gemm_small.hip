@@ -18,11 +18,13 @@
 // barrier publishes that stage and frees this one's slot for the loads of stage kt + NSLOT.
 //
 // fp32 operands run here at every size (v_mfma_f32_32x32x2_f32, a stage of 32 floats per row,
-// lane half h of a fragment taking floats 16 h .. 16 h + 15 in turn): each stage is 4096 cycles of
-// MFMA per SIMD for 32 KB, so the matrix cores are the bound, and the ring with one barrier per
-// stage and fragments read a step ahead keeps them fed where the register-staged kernel
-// (gemm_f32.hip, which the convolutions still use, with the same K order and so the same bits)
-// reached two thirds of their rate: UMT5's four linears of 452 rows 1936 -> F32SUM us.
+// lane half h of a fragment taking floats 16 h .. 16 h + 15 in turn), bound by the matrix cores:
+// 128 x 128 takes 4096 cycles of MFMA per SIMD and stage for 32 KB. What keeps them fed is other
+// workgroups on the unit while one is at its barrier, so these tiles take two slots of a ring
+// each (two workgroups per unit at 128 x 128, five at 64 x 64): four linears of 452 rows (4096 x
+// 12288, 4096 x 4096, 4096 x 20480, 10240 x 4096) 1867 us in the register-staged kernel
+// (gemm_f32.hip, which the convolutions still use, with the same K order and so the same bits),
+// 1667 with rings of 4 and 5 slots, 1510 now; 1024 rows of 4096 x 12288 897 -> 749 us (138 TFLOP/s).
 //
 // K pieces: piece c of a tile writes its fp32 sums to part[c][m][n]; gemm_small_reduce adds the
 // pieces in order and runs the epilogue. Nothing is kept between launches and nobody waits, so
@@ -143,20 +145,22 @@ __device__ __forceinline__ void small_store8(const SmallArgs& a, int64_t m, int6
 }
 
 template <SmallElem E, int BM, int BN, int NSLOT, bool GATE>
-__global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args) {
+__global__ __launch_bounds__(BN == 64 ? 256 : 512, 1) void gemm_small_kernel(
+    const SmallArgs args) {
   constexpr bool F32 = E == SmallElem::F32;
   constexpr int EB = F32 ? 4 : E == SmallElem::BF16 ? 2 : 1;
-  constexpr int WAVES_M = BM == 256 ? 4 : 2, WAVES_N = 8 / WAVES_M;
+  constexpr int NW = BN == 64 ? 4 : 8, NT = NW * 64;  // wavefronts, threads
+  constexpr int WAVES_M = BM == 256 ? 4 : 2, WAVES_N = NW / WAVES_M;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int TI = WTM / 32, TJ = WTN / 32;     // MFMA tiles per wave
   constexpr int NKS = EB > 1 ? 4 : 2;  // K steps per stage (F32: of 4 MFMAs each)
   constexpr int NA = EB > 1 ? 1 : 2;   // 16-byte LDS reads per fragment
-  constexpr int SA = BM / 64, SW = BN / 64, LPS = SA + SW;  // 1 KB loads per wave and stage
+  constexpr int SA = BM / 8 / NW, SW = BN / 8 / NW, LPS = SA + SW;  // 1 KB loads per wave and stage
   constexpr int SLOT = (BM + BN) * 128;
   // MX: E8M0 scales of 4 stages (16 bytes) per row, a ring of two such blocks
   constexpr int SC = E == SmallElem::MX ? (BM + BN) * 16 : 0;
   static_assert(NSLOT * SLOT >= BM * BN * 4, "the epilogue stages the fp32 tile in the ring");
-  static_assert(NSLOT >= 3 && NSLOT <= 5, "scale blocks land within 4 stages");
+  static_assert(E != SmallElem::MX || NSLOT <= 5, "scale blocks land within 4 stages");
   __shared__ __attribute__((aligned(16))) uint8_t lds[NSLOT * SLOT + 2 * SC];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -355,11 +359,12 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
     st = nst;
   }
 
-  // ---- the fp32 tile through the idle ring: 16-byte chunk c of row r at c ^ (r & 31), then
+  // ---- the fp32 tile through the idle ring: 16-byte chunk c of row r at c ^ (r & CM), then
   // BN / 8 lanes per row take 8 columns each (whole lines per store)
   wait_vm<0>();
   __syncthreads();
   float* tile = reinterpret_cast<float*>(lds);
+  constexpr int CM = BN / 4 < 32 ? BN / 4 - 1 : 31;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -370,20 +375,20 @@ __global__ __launch_bounds__(512, 1) void gemm_small_kernel(const SmallArgs args
         const int c4 = (wn * WTN + j * 32 + q * 8 + fhalf * 4) >> 2;
         const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                          acc[i][j][4 * q + 3]};
-        *reinterpret_cast<f32x4*>(tile + r * BN + ((c4 ^ (r & 31)) << 2)) = v;
+        *reinterpret_cast<f32x4*>(tile + r * BN + ((c4 ^ (r & CM)) << 2)) = v;
       }
     }
   __syncthreads();
-  constexpr int LPR = BN / 8, RPP = 512 / LPR;  // lanes per row, rows per pass
+  constexpr int LPR = BN / 8, RPP = NT / LPR;  // lanes per row, rows per pass
   const int ch = tid % LPR, rsub = tid / LPR;
   const int64_t n = n0 + ch * 8;
 #pragma unroll 4
   for (int r = rsub; r < BM; r += RPP) {
     const int64_t m = m0 + r;
     if (m >= M) break;
-    const f32x4 y0 = *reinterpret_cast<const f32x4*>(tile + r * BN + (((2 * ch) ^ (r & 31)) << 2));
+    const f32x4 y0 = *reinterpret_cast<const f32x4*>(tile + r * BN + (((2 * ch) ^ (r & CM)) << 2));
     const f32x4 y1 =
-        *reinterpret_cast<const f32x4*>(tile + r * BN + (((2 * ch + 1) ^ (r & 31)) << 2));
+        *reinterpret_cast<const f32x4*>(tile + r * BN + (((2 * ch + 1) ^ (r & CM)) << 2));
     if (args.pieces > 1) {
       float* p = args.part + ((int64_t)piece * M + m) * N + n;
       if (n < N) *reinterpret_cast<f32x4*>(p) = y0;
@@ -420,9 +425,12 @@ __global__ __launch_bounds__(256) void gemm_small_reduce(const SmallArgs args) {
 }
 
 // Estimated times on MI355X, in us, from sweeps over 16 to 3000 rows of the layers' widths:
-//  - a workgroup takes kStage per K stage (bf16, fp8, MXFP8, fp32; 64-, 128- and 256-row tiles;
-//    the MX scales cost the small tiles LDS reads, fp32 is the MFMAs' time) plus 5 for its first loads and its output; a launch runs
+//  - a workgroup takes kStage per K stage (bf16, fp8, MXFP8; 64-, 128- and 256-row tiles; the MX
+//    scales cost the small tiles LDS reads) plus 5 for its first loads and its output; a launch runs
 //    ceil(workgroups / units) rounds of that, but no faster than its weights come from HBM;
+//  - fp32 (64 x 64 and 128 x 128 tiles): a compute unit works through its workgroups' stages two
+//    or more workgroups at a time, kStageF32 each with one, two or more of them on the unit
+//    (matrix-core time 0.43 and 1.74 at 2.35 GHz);
 //  - cutting K adds the reduce launch and the sums' trip out and back at about 5 TB/s.
 // 16 and 8 rows apart from the boundary the choices measured (bf16, K = N = 3072 / 12288 x 3072 /
 // 5120 x 5120, 256 x 256 tiles -> the plan's): 64 rows 57 -> 16, 65 -> 23, 50 -> 18; 512 rows
@@ -438,24 +446,27 @@ SmallPlan small_plan(SmallElem e, int64_t m, int64_t n, int64_t k, int cus, int6
   const int nk = (int)((k * eb + 127) / 128), gran = e == SmallElem::MX ? 4 : 1;
   // PLAN
   static const int kRows[3] = {64, 128, 256};
-  static const double kStage[4][3] = {
-      {0.36, 0.52, 0.90}, {0.30, 0.43, 0.88}, {0.38, 0.60, 0.90}, {0.90, 1.78, 3.55}};
+  static const double kStage[3][3] = {{0.36, 0.52, 0.90}, {0.30, 0.43, 0.88}, {0.38, 0.60, 0.90}};
+  static const double kStageF32[2][3] = {{0.62, 0.53, 0.505}, {2.05, 1.95, 1.93}};
   const double hbm_us = (double)n * k * eb / 4.5e6;
   double best_us = 0.95 * big_us;  // within the estimates' error of each other: leave it
-  for (int i = 0; i < 3; ++i) {
-    const int64_t tiles = ((m + kRows[i] - 1) / kRows[i]) * ((n + 127) / 128);
+  for (int i = 0; i < (f32 ? 2 : 3); ++i) {
+    const int bn = f32 && i == 0 ? 64 : 128;
+    const int64_t tiles = ((m + kRows[i] - 1) / kRows[i]) * ((n + bn - 1) / bn);
     if (tiles > 4 * cus && !f32) continue;
     for (int pieces = 1; pieces <= 16; ++pieces) {
       const int ps = ((nk + pieces - 1) / pieces + gran - 1) / gran * gran;
       if ((nk + ps - 1) / ps != pieces) continue;  // rounding left a piece without stages
       if (pieces > 1 && (ps < 4 || pieces * m * n * 4 > scratch)) continue;
       if (pieces > 1 && tiles * pieces > 4 * cus) break;
-      const double rounds = (double)((tiles * pieces + cus - 1) / cus);
-      double us = std::max(rounds * (ps * kStage[(int)e][i] + 5.0), hbm_us);
+      const int64_t rounds = (tiles * pieces + cus - 1) / cus;
+      double us = f32 ? rounds * ps * kStageF32[i][std::min<int64_t>(rounds, 3) - 1] + 5.0
+                      : rounds * (ps * kStage[(int)e][i] + 5.0);
+      us = std::max(us, hbm_us);
       if (pieces > 1) us += 3.0 + (double)pieces * m * n * 8 / 5e6;
       if (us < best_us) {
         best_us = us;
-        best = {kRows[i], 128, pieces, ps};
+        best = {kRows[i], bn, pieces, ps};
       }
     }
   }
@@ -465,12 +476,19 @@ SmallPlan small_plan(SmallElem e, int64_t m, int64_t n, int64_t k, int cus, int6
 template <SmallElem E, bool GATE>
 static void launch_small(const SmallArgs& a, const SmallPlan& p, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n * a.pieces)), block(512);
-  if (p.bm == 64)
-    hipLaunchKernelGGL((gemm_small_kernel<E, 64, 128, 5, GATE>), grid, block, 0, s, a);
-  else if (p.bm == 128)
-    hipLaunchKernelGGL((gemm_small_kernel<E, 128, 128, 4, GATE>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((gemm_small_kernel<E, 256, 128, 3, GATE>), grid, block, 0, s, a);
+  if constexpr (E == SmallElem::F32) {
+    if (p.bm == 64)
+      hipLaunchKernelGGL((gemm_small_kernel<E, 64, 64, 2, GATE>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((gemm_small_kernel<E, 128, 128, 2, GATE>), grid, block, 0, s, a);
+  } else {
+    if (p.bm == 64)
+      hipLaunchKernelGGL((gemm_small_kernel<E, 64, 128, 5, GATE>), grid, block, 0, s, a);
+    else if (p.bm == 128)
+      hipLaunchKernelGGL((gemm_small_kernel<E, 128, 128, 4, GATE>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((gemm_small_kernel<E, 256, 128, 3, GATE>), grid, block, 0, s, a);
+  }
   if (p.pieces > 1) {
     const int64_t chunks = (int64_t)a.m * ((a.n + 7) / 8);
     hipLaunchKernelGGL((gemm_small_reduce<E, GATE>), dim3((unsigned)((chunks + 255) / 256)),
