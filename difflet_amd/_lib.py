@@ -85,6 +85,8 @@ SIGNATURES: dict[str, tuple] = {
     "difflet_rocm_gemm_f32_scratch": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64,
                                              _i64, _i64, _i64, _vp, _i64, _vp]),
     "difflet_rocm_gemm_scratch_bytes": (_i64, [_i32, _i64, _i64, _i64]),
+    "difflet_rocm_gemm_single": (_i32, [_i32, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64,
+                                        _i64, _i64, _vp, _i64, _vp]),
     "difflet_rocm_gemm_bf16": (_i32, [_i32, ctypes.POINTER(GemmProblem), _i64, _i64, _i32,
                                       _i64, _vp, _i64, ctypes.POINTER(GemmQk), _vp]),
     "difflet_rocm_gemm_fp8_rowwise": (_i32, [_i32, ctypes.POINTER(GemmProblem), _i64, _i64,

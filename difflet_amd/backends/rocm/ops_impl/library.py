@@ -7,6 +7,12 @@ Inductor compiles the torch code around them. This is what the reference's CUDA 
 do for their own fused kernels (difflet/backends/cuda/hunyuan_video_15/modeling.py:73-100,
 difflet/backends/tpu/ops_impl/collectives.py:99-150).
 
+A custom_op's Python layers cost about 10 us a call, as much as a short linear on the device. So
+the operators of the linears and the attention each have a twin, ``<name>_infer``, with the same
+implementation and fake but a bare dispatcher registration; the functions here call the twin for
+device tensors that need no gradient, outside torch.compile. Everything else (graphs, inputs that
+require grad, whose backward custom_op refuses, host tensors) goes to the custom_op.
+
 Every operator is functional: it allocates and returns a new contiguous tensor and mutates no
 argument. Shape and dtype checks that raise for unsupported inputs stay in the op modules, so
 they also run while tracing.
@@ -23,34 +29,78 @@ from difflet_amd import kernels
 
 Tensor = torch.Tensor
 
+_INFER = torch.library.Library("difflet_rocm", "FRAGMENT")  # noqa: TOR901
+
+
+def _infer_twin(op, impl, fake):
+    """The operator <op's name>_infer of op's signature: impl on the device, fake for tracing."""
+    schema = op._opoverload._schema
+    name = schema.name.split("::")[1]
+    _INFER.define(str(schema).split("::")[1].replace(f"{name}(", f"{name}_infer(", 1))
+    _INFER.impl(f"{name}_infer", impl, "CUDA")
+    torch.library.register_fake(f"difflet_rocm::{name}_infer", fake, lib=_INFER)
+    return getattr(torch.ops.difflet_rocm, f"{name}_infer").default
+
+
+def _plain(*tensors: Optional[Tensor]) -> bool:
+    """Device tensors, none of which needs a gradient."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (not t.is_cuda or (grad and t.requires_grad)):
+            return False
+    return True
+
 
 # ---------------------------------------------------------------------------------- attention
-@torch.library.custom_op("difflet_rocm::attention", mutates_args=())
-def attention(q: Tensor, k: Tensor, v: Tensor, scale: float, causal: bool,
-              attention_mask: Optional[Tensor], bound_min: Optional[Tensor],
-              bound_max: Optional[Tensor]) -> Tensor:
+def _attention_impl(q: Tensor, k: Tensor, v: Tensor, scale: float, causal: bool,
+                    attention_mask: Optional[Tensor], bound_min: Optional[Tensor],
+                    bound_max: Optional[Tensor]) -> Tensor:
     """difflet_rocm_attention: (B, H, S, D) or (B*H, S, D) q/k/v, output in v's dtype."""
     return kernels.attention(q, k, v, scale=scale, causal=causal, attention_mask=attention_mask,
                              bound_min=bound_min, bound_max=bound_max).contiguous()
 
 
-@attention.register_fake
-def _(q, k, v, scale, causal, attention_mask, bound_min, bound_max):
+def _attention_fake(q, k, v, scale, causal, attention_mask, bound_min, bound_max):
     return q.new_empty((*q.shape[:-1], v.shape[-1]), dtype=v.dtype)
 
 
-@torch.library.custom_op("difflet_rocm::attention_joint", mutates_args=())
-def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
-                    key_count: Optional[Tensor], count_offset: int) -> Tensor:
+_attention_op = torch.library.custom_op("difflet_rocm::attention", _attention_impl, mutates_args=())
+_attention_op.register_fake(_attention_fake)
+_attention_infer = _infer_twin(_attention_op, _attention_impl, _attention_fake)
+
+
+def attention(q: Tensor, k: Tensor, v: Tensor, scale: float, causal: bool,
+              attention_mask: Optional[Tensor], bound_min: Optional[Tensor],
+              bound_max: Optional[Tensor]) -> Tensor:
+    if not torch.compiler.is_compiling() and _plain(q, k, v, attention_mask, bound_min, bound_max):
+        return _attention_infer(q, k, v, scale, causal, attention_mask, bound_min, bound_max)
+    return _attention_op(q, k, v, scale, causal, attention_mask, bound_min, bound_max)
+
+
+def _attention_joint_impl(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
+                          key_count: Optional[Tensor], count_offset: int) -> Tensor:
     """difflet_rocm_attention_joint: (B, H, S, 128) q over the keys [k | k2], the first
     key_count[b] + count_offset of them when key_count is given."""
     return kernels.attention_joint(q, k, v, k2, v2, scale=scale, key_count=key_count,
                                    count_offset=count_offset)
 
 
-@attention_joint.register_fake
-def _(q, k, v, k2, v2, scale, key_count, count_offset):
+def _attention_joint_fake(q, k, v, k2, v2, scale, key_count, count_offset):
     return q.new_empty(q.shape)
+
+
+_attention_joint_op = torch.library.custom_op("difflet_rocm::attention_joint",
+                                              _attention_joint_impl, mutates_args=())
+_attention_joint_op.register_fake(_attention_joint_fake)
+_attention_joint_infer = _infer_twin(_attention_joint_op, _attention_joint_impl,
+                                     _attention_joint_fake)
+
+
+def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
+                    key_count: Optional[Tensor], count_offset: int) -> Tensor:
+    if not torch.compiler.is_compiling() and _plain(q, k, v, k2, v2, key_count):
+        return _attention_joint_infer(q, k, v, k2, v2, scale, key_count, count_offset)
+    return _attention_joint_op(q, k, v, k2, v2, scale, key_count, count_offset)
 
 
 # ------------------------------------------------------------------------------------- linear
@@ -63,8 +113,7 @@ def _gemv_fits(m: int, k: int) -> bool:
     return m <= GEMV_ROWS and k % 8 == 0 and {1: 1, 2: 2}.get(m, 4 if m <= 4 else 8) * k <= 16384
 
 
-@torch.library.custom_op("difflet_rocm::linear", mutates_args=())
-def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
+def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
     """y [M, out_features] bf16 = x [M, K'] @ w[:out_features, :K']^T + bias, where w [N', K'] may be
     the zero-padded weight (K' a multiple of 64, N' of 4); x is padded to K' here."""
     m, kx = x.shape
@@ -77,17 +126,26 @@ def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> T
         x = F.pad(x, (0, k_pad - kx))
     if bias is not None and bias.shape[0] != n_pad:
         bias = F.pad(bias, (0, n_pad - bias.shape[0]))
-    y = kernels.linear(x if x.stride(-1) == 1 else x.contiguous(), w, bias, workspace="call")
+    y = kernels.gemm_call("bf16", x if x.stride(-1) == 1 else x.contiguous(), w, bias)
     return y if n_pad == out_features else y[:, :out_features].contiguous()
 
 
-@linear.register_fake
-def _(x, w, bias, out_features):
+def _linear_fake(x, w, bias, out_features):
     return x.new_empty((x.shape[0], out_features), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("difflet_rocm::linear_f32", mutates_args=())
-def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
+_linear_op = torch.library.custom_op("difflet_rocm::linear", _linear_impl, mutates_args=())
+_linear_op.register_fake(_linear_fake)
+_linear_infer = _infer_twin(_linear_op, _linear_impl, _linear_fake)
+
+
+def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
+    if not torch.compiler.is_compiling() and _plain(x, w, bias):
+        return _linear_infer(x, w, bias, out_features)
+    return _linear_op(x, w, bias, out_features)
+
+
+def _linear_f32_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
     """y [M, out_features] fp32 = x [M, K'] @ w[:out_features, :K']^T + bias on the fp32 GEMM,
     where w [N', K'] may be the zero-padded weight (K' and N' multiples of 4)."""
     m, kx = x.shape
@@ -103,29 +161,48 @@ def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) 
     return y if n_pad == out_features else y[:, :out_features].contiguous()
 
 
-@linear_f32.register_fake
-def _(x, w, bias, out_features):
+def _linear_f32_fake(x, w, bias, out_features):
     return x.new_empty((x.shape[0], out_features), dtype=torch.float32)
 
 
-@torch.library.custom_op("difflet_rocm::fp8_linear", mutates_args=())
-def fp8_linear(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
+_linear_f32_op = torch.library.custom_op("difflet_rocm::linear_f32", _linear_f32_impl,
+                                         mutates_args=())
+_linear_f32_op.register_fake(_linear_f32_fake)
+_linear_f32_infer = _infer_twin(_linear_f32_op, _linear_f32_impl, _linear_f32_fake)
+
+
+def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
+    if not torch.compiler.is_compiling() and _plain(x, w, bias):
+        return _linear_f32_infer(x, w, bias, out_features)
+    return _linear_f32_op(x, w, bias, out_features)
+
+
+def _fp8_linear_impl(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
                mx: bool) -> Tensor:
     """The fp8 twins' matmul: x [M, K] bf16 quantized per token (per-channel weights) or per MX
     block in swizzle order (mx), then the fp8 GEMM with fp32 accumulation, bf16 [M, N] out."""
-    y = torch.empty((x.shape[0], w_kernel.shape[0]), dtype=torch.bfloat16, device=x.device)
     if mx:
         aq, asc = kernels.quantize_mxfp8(x, swizzled=True)
     else:
         aq, asc = kernels.quantize_fp8_rowwise(x)
-    kernels.gemm_grouped([kernels.Problem(aq, w_kernel, y, bias, a_scale=asc, w_scale=w_scale)],
-                         kind="mx" if mx else "fp8", workspace="call")
-    return y
+    return kernels.gemm_call("mx" if mx else "fp8", aq, w_kernel, bias, asc, w_scale)
 
 
-@fp8_linear.register_fake
-def _(x, w_kernel, w_scale, bias, mx):
+def _fp8_linear_fake(x, w_kernel, w_scale, bias, mx):
     return x.new_empty((x.shape[0], w_kernel.shape[0]), dtype=torch.bfloat16)
+
+
+_fp8_linear_op = torch.library.custom_op("difflet_rocm::fp8_linear", _fp8_linear_impl,
+                                         mutates_args=())
+_fp8_linear_op.register_fake(_fp8_linear_fake)
+_fp8_linear_infer = _infer_twin(_fp8_linear_op, _fp8_linear_impl, _fp8_linear_fake)
+
+
+def fp8_linear(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
+               mx: bool) -> Tensor:
+    if not torch.compiler.is_compiling() and _plain(x, w_kernel, w_scale, bias):
+        return _fp8_linear_infer(x, w_kernel, w_scale, bias, mx)
+    return _fp8_linear_op(x, w_kernel, w_scale, bias, mx)
 
 
 # ---------------------------------------------------------------------------- norms, rotary

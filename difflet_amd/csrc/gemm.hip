@@ -1297,6 +1297,30 @@ extern "C" int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t 
   return p.pieces > 1 ? SK_CTR_BYTES + p.pieces * m * n * 4 : 0;
 }
 
+extern "C" int difflet_rocm_gemm_single(int kind, const void* a, int64_t lda, const void* w,
+                                        int64_t ldw, void* c, int64_t ldc, const void* bias,
+                                        const void* a_scale, const void* w_scale, int64_t m,
+                                        int64_t n, int64_t k, void* workspace,
+                                        int64_t workspace_bytes, difflet_stream_t stream) {
+  difflet_gemm_problem q = {};
+  q.a = a;
+  q.lda = lda;
+  q.w = w;
+  q.ldw = ldw;
+  q.c = c;
+  q.ldc = ldc;
+  q.bias = bias;
+  q.a_scale = a_scale;
+  q.w_scale = w_scale;
+  q.m = m;
+  q.rows_per_batch = m;
+  DLT_REQUIRE(kind >= 0 && kind <= 2, DIFFLET_EINVAL, "gemm_single: unknown kind %d", kind);
+  auto* fn = kind == 0   ? difflet_rocm_gemm_bf16
+             : kind == 1 ? difflet_rocm_gemm_fp8_rowwise
+                         : difflet_rocm_gemm_mxfp8;
+  return fn(1, &q, n, k, DIFFLET_EPI_NONE, 0, workspace, workspace_bytes, nullptr, stream);
+}
+
 extern "C" int difflet_rocm_gemm_bf16(int nproblems, const difflet_gemm_problem* problems,
                                       int64_t n, int64_t k, int epilogue,
                                       int64_t act_col_start, void* workspace,

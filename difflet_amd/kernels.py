@@ -42,8 +42,13 @@ def _ptr(t: torch.Tensor | None):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _raw_stream(dev: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(
+        dev.index if dev.index is not None else torch.cuda.current_device())
+
+
 def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return ctypes.c_void_p(_raw_stream(dev))
 
 
 def _on_gpu(*ts: torch.Tensor | None) -> torch.device:
@@ -459,6 +464,54 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
     fn = getattr(lib(), _GEMM_FN[kind])
     check(fn(len(problems), arr, n, k, int(epilogue), int(act_col_start), ws_ptr, ws_bytes,
              qk_arg, _stream(dev)), f"gemm_{kind}")
+
+
+_GEMM_A_DTYPES = {"bf16": (torch.bfloat16,), "fp8": (torch.float8_e4m3fn, torch.uint8),
+                  "mx": (torch.float8_e4m3fn, torch.uint8)}
+
+
+def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None,
+              a_scale: torch.Tensor | None = None, w_scale: torch.Tensor | None = None
+              ) -> torch.Tensor:
+    """bf16 [M, N] = A W^T + bias, one problem without an epilogue: gemm_grouped with workspace
+    "call" in a third of its host time (short prompts spend more on the host than on the device:
+    16 rows of 3072 x 3072 took 37 us a call, 23 now). Operands in the plain form below go
+    straight to the library; any other goes to gemm_grouped, which refuses or runs it."""
+    m, k = a.shape[0], w.shape[-1]
+    n = w.shape[0]
+    dev = a.device
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    kid = _KIND_ID[kind]
+
+    def vec(t, dtype, length):
+        return (t.dtype is dtype and t.device == dev and t.dim() == 1 and t.shape[0] >= length
+                and t.stride(0) == 1)
+
+    dts = _GEMM_A_DTYPES[kind]
+    plain = (m > 0 and a.is_cuda and w.device == dev and a.dim() == 2 and w.dim() == 2
+             and a.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1
+             and a.dtype in dts and w.dtype in dts and (bias is None or vec(bias, torch.bfloat16, n)))
+    if kid == 1:
+        plain = (plain and a_scale is not None and w_scale is not None
+                 and vec(a_scale, torch.float32, m) and vec(w_scale, torch.float32, n))
+    elif kid == 2:
+        plain = plain and all(
+            t is not None and t.dtype is torch.uint8 and t.device == dev
+            and t.shape == (rows, k // 32) and t.is_contiguous()
+            for t, rows in ((a_scale, m), (w_scale, n)))
+    if not plain:
+        gemm_grouped([Problem(a, w, y, bias, a_scale=a_scale, w_scale=w_scale)], kind=kind,
+                     workspace="call")
+        return y
+    c = lib()
+    nbytes = c.difflet_rocm_gemm_scratch_bytes(kid, m, n, k)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    check(c.difflet_rocm_gemm_single(
+        kid, a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), n,
+        None if bias is None else bias.data_ptr(), a_scale.data_ptr() if kid else None,
+        w_scale.data_ptr() if kid else None, m, n, k, None if ws is None else ws.data_ptr(), nbytes,
+        _raw_stream(dev)), f"gemm_{kind}")
+    return y
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,

@@ -242,6 +242,13 @@ int64_t difflet_rocm_gemm_workspace_bytes(void);
  * needs zeroed counters. */
 int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k);
 
+/* One problem with EPI_NONE through the GEMM of `kind` (0 bf16, 1 fp8 per row, 2 MXFP8), its
+ * operands as plain arguments. */
+int difflet_rocm_gemm_single(int kind, const void* a, int64_t lda, const void* w, int64_t ldw,
+                             void* c, int64_t ldc, const void* bias, const void* a_scale,
+                             const void* w_scale, int64_t m, int64_t n, int64_t k,
+                             void* workspace, int64_t workspace_bytes, difflet_stream_t stream);
+
 /* bf16 x bf16 -> fp32 accumulate -> bf16. k % 64 == 0. */
 int difflet_rocm_gemm_bf16(int nproblems, const difflet_gemm_problem* problems, int64_t n,
                            int64_t k, int epilogue, int64_t act_col_start, void* workspace,

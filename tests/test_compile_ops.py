@@ -82,3 +82,24 @@ def test_compile_options_extend_the_mode():
     blocks = nn.ModuleList([nn.Linear(2, 2)])
     assert rc.compile_blocks([blocks], dynamic=False, options={"max_autotune": False}) == 1
     assert rc.COMPILE_MODE == "max-autotune-no-cudagraphs"
+
+
+def test_infer_twins_mirror_the_custom_ops():
+    """The twin that eager inference calls: same signature, same fake; not taken for host tensors
+    or tensors that require grad."""
+    ops = torch.ops.difflet_rocm
+    for name in ("attention", "attention_joint", "linear", "linear_f32", "fp8_linear"):
+        a = getattr(ops, name).default._schema
+        b = getattr(ops, f"{name}_infer").default._schema
+        assert str(a).split("(", 1)[1] == str(b).split("(", 1)[1]
+    with FakeTensorMode():
+        x = torch.empty(33, 384, dtype=torch.bfloat16, device="cuda")
+        w = torch.empty(100, 384, dtype=torch.bfloat16, device="cuda")
+        assert library._plain(x, w, None) and not library._plain(x, w.requires_grad_())
+        with torch.no_grad():
+            assert library._plain(x, w)
+        assert not library._plain(torch.empty(3))
+        y = library.linear(x, w, None, 99)  # w requires grad: the custom op
+        assert y.shape == (33, 99) and y.requires_grad
+        y = library.linear(x, w.detach(), None, 99)
+        assert y.shape == (33, 99) and y.dtype == torch.bfloat16 and y.is_cuda
