@@ -69,9 +69,13 @@ __global__ __launch_bounds__(512, 1) void conv_igemm_kernel(const ConvArgs a) {
   constexpr int SW = BN / 8;   // W slabs per stage, wave w taking w, w + 8, ...
   constexpr int NWJ = (SW + 7) / 8;
   constexpr int SLOT = (BM + BN) * 128;
-  static_assert(SA % 2 == 0 && SA <= 8 && NWJ <= 3 && NJ <= 3 && 2 * SLOT <= 160 * 1024,
+  // a third stage slot where it fits (256 x 128): two stages in flight behind the one computed
+  // (128 channels at 1024 x 1024: 466 -> 430 us; a tile costs 1.1 us a stage, 1.2 before, and
+  // about 7 for its first loads and its output)
+  constexpr int NSLOT = 3 * SLOT <= 160 * 1024 && SW % 8 == 0 ? 3 : 2;
+  static_assert(SA % 2 == 0 && SA <= 8 && NWJ <= 3 && NJ <= 3 && NSLOT * SLOT <= 160 * 1024,
                 "tile does not fit the LDS");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * SLOT];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[NSLOT * SLOT];
   typedef __attribute__((address_space(3))) void lds_void;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -244,31 +248,38 @@ __global__ __launch_bounds__(512, 1) void conv_igemm_kernel(const ConvArgs a) {
                                                           acc[i][j], 0, 0, 0);
   };
 
-  // Stage 0 lands before the loop; stage kt + 1 is in flight while stage kt computes. Before the
-  // last K step of stage kt every wave waits for its loads (stage kt + 1's, the only ones in
-  // flight) and its LDS reads, and one barrier publishes stage kt + 1 and frees slot kt & 1 for
-  // stage kt + 2, whose loads go out with the last K step's MFMAs.
-  issue_part(kbeg, 0, 0);
-  issue_part(kbeg, 0, 1);
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  // Stages kt + 1 .. kt + NSLOT - 1 are in flight while stage kt computes. Before the last K step
+  // of stage kt every wave waits for its loads of stage kt + 1 (with three slots those of stage
+  // kt + 2, SA + NWJ of them, may stay in flight) and its LDS reads, and one barrier publishes
+  // stage kt + 1 and frees the slot of stage kt for stage kt + NSLOT, whose loads go out with the
+  // last K step's MFMAs.
+  constexpr int YOUNGER = SA + NWJ;
+#pragma unroll
+  for (int s = 0; s < NSLOT; ++s)
+    if (kbeg + s < kend) {
+      issue_part(kbeg + s, s, 0);
+      issue_part(kbeg + s, s, 1);
+      // the first stage lands before the loop; waiting for it first keeps the count simple
+      if (s == 0) __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    }
   __syncthreads();
-  if (kend - kbeg > 1) {
-    issue_part(kbeg + 1, 1, 0);
-    issue_part(kbeg + 1, 1, 1);
-  }
   read_w(0, 0, 0);
   read_a(0, 0, 0);
   read_a(0, 0, 1);
+  int st = 0;
   for (int kt = kbeg; kt < kend; ++kt) {
-    const int st = (kt - kbeg) & 1;
+    const int nxt = st == NSLOT - 1 ? 0 : st + 1;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int set = ks & 1;
       const bool last = ks == 3;
-      const int nst = last ? (st ^ 1) : st, nks = last ? 0 : ks + 1;
-      const bool loads = last && kt + 2 < kend;
+      const int nst = last ? nxt : st, nks = last ? 0 : ks + 1;
+      const bool loads = last && kt + NSLOT < kend;
       if (last) {
-        __builtin_amdgcn_s_waitcnt(0x0070);
+        if (NSLOT == 3 && kt + 2 < kend)
+          __builtin_amdgcn_s_waitcnt(0x0070 | YOUNGER);
+        else
+          __builtin_amdgcn_s_waitcnt(0x0070);
         asm volatile("s_barrier" ::: "memory");
       }
       read_w(nst, nks, set ^ 1);
@@ -276,11 +287,13 @@ __global__ __launch_bounds__(512, 1) void conv_igemm_kernel(const ConvArgs a) {
       for (int i = 0; i < 2; ++i) {
         mma_tile(set, i);
         read_a(nst, nks, i);
-        if (loads) issue_part(kt + 2, st, i);
+        if (loads) issue_part(kt + NSLOT, st, i);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    st = nxt;
   }
+  static_assert(YOUNGER < 16, "vmcnt field");
 
   // ---- epilogue: lane holds pixel m0 + wm 64 + 32 i + (lane & 31) and, per group g, the four
   // channels 8 g + 4 (lane >> 5) .. + 3 of each 32-channel tile: + bias (+ residual), rounded once
@@ -370,12 +383,22 @@ namespace {
 
 // The tile for n output channels, as (WMW, NJ): the widest that wastes little, 512 x 32 NJ up to
 // 96 channels, 256 x 128 up to 128, then 256 x 192 unless rounding up to 192 adds over an eighth
-// (256 channels: two 256 x 128).
-void conv_tile(int64_t n, int& wmw, int& nj) {
+// (256 channels: two 256 x 128) or its last wave of tiles is so empty that 256 x 128 ends sooner
+// (512 channels over 128 x 128 pixels: 192 tiles of 256 x 192 102 us, 256 of 256 x 128 78; over
+// 256 x 256 pixels 325 both ways). A wave takes 1.42 us per K stage of a 192-wide tile, 1.08 of a
+// 128-wide one, and 7. Launches of under half a wave of wide tiles keep them and cut K (conv_plan).
+void conv_tile(int64_t rows, int64_t n, int64_t nk, int cus, int& wmw, int& nj) {
+  const int64_t tm = (rows + 255) / 256;
+  auto us = [&](int64_t bn, double stage) {
+    const int64_t waves = (tm * ((n + bn - 1) / bn) + cus - 1) / cus;
+    return (double)waves * ((double)nk * stage + 7.0);
+  };
   if (n <= 96) {
     wmw = 8;
     nj = (int)((n + 31) / 32);
-  } else if (n <= 128 || (n + 191) / 192 * 192 * 8 > 9 * n) {
+  } else if (n <= 128 || (n + 191) / 192 * 192 * 8 > 9 * n ||
+             (2 * tm * ((n + 191) / 192) >= cus && cus > 0 &&
+              us(128, 1.08) < 0.95 * us(192, 1.42))) {
     wmw = 4;
     nj = 2;
   } else {
@@ -408,7 +431,7 @@ struct ConvPlan {
 // one wave of workgroups runs; the ranges' fp32 partial sums meet in a second kernel.
 ConvPlan conv_plan(int64_t rows, int64_t n, int64_t kpad, int cus) {
   ConvPlan p;
-  conv_tile(n, p.wmw, p.nj);
+  conv_tile(rows, n, kpad / 64, cus, p.wmw, p.nj);
   const int bm = 64 * p.wmw, bn = 32 * p.nj * (8 / p.wmw);
   p.tiles_n = (int)((n + bn - 1) / bn);
   p.tiles = (rows + bm - 1) / bm * p.tiles_n;
