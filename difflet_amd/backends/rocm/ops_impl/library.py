@@ -104,13 +104,16 @@ def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, sca
 
 
 # ------------------------------------------------------------------------------------- linear
-#: up to this many input rows a linear runs on the GEMV kernel (HBM-bound on the weight)
+#: up to this many input rows a linear may run on the GEMV kernel (HBM-bound on the weight)
 GEMV_ROWS = 8
 
 
-def _gemv_fits(m: int, k: int) -> bool:
-    """The GEMV kernel stages m rows of x in LDS: m (rounded up to 1, 2, 4 or 8) x k <= 16384."""
-    return m <= GEMV_ROWS and k % 8 == 0 and {1: 1, 2: 2}.get(m, 4 if m <= 4 else 8) * k <= 16384
+def _gemv_fits(m: int, k: int, n: int) -> bool:
+    """The GEMV kernel stages m rows of x in LDS: m (rounded up to 1, 2, 4 or 8) x k <= 16384. From
+    two rows on its reads of x bound it (3072 x 18432: 2 rows 34 us, 4 rows 56, the GEMM's 64-row
+    tiles 26), so there it keeps the widths the GEMM would have to pad the weight for."""
+    return (m <= GEMV_ROWS and k % 8 == 0 and (m == 1 or k % 64 != 0 or n % 4 != 0)
+            and {1: 1, 2: 2}.get(m, 4 if m <= 4 else 8) * k <= 16384)
 
 
 def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
@@ -120,7 +123,7 @@ def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int
     n_pad, k_pad = w.shape
     if m == 0:
         return x.new_empty((0, out_features), dtype=torch.bfloat16)
-    if n_pad == out_features and k_pad == kx and _gemv_fits(m, kx):
+    if n_pad == out_features and k_pad == kx and _gemv_fits(m, kx, n_pad):
         return kernels.gemv(x, w, bias)
     if kx != k_pad:
         x = F.pad(x, (0, k_pad - kx))

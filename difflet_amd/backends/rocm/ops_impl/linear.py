@@ -6,8 +6,9 @@ Same constructors, attributes, state dicts and bias semantics as the CPU twins
 ``(x @ W^T, bias)``; ``reduce_output`` / ``gather_output`` / ``input_is_parallel`` /
 ``reduce_dtype`` are accepted and have no effect at tp = 1.
 
-The matmul: bf16 weights run the bf16 kernels, up to 8 rows of input through the GEMV kernel
-(the modulation and timestep linears, HBM-bound on W), more through the tiled GEMM; fp32
+The matmul: bf16 weights run the bf16 kernels, one row of input (up to 8 at widths the GEMM would
+pad) through the GEMV kernel (the modulation and timestep linears, HBM-bound on W), more through
+the tiled GEMM; fp32
 weights (a model loaded in fp32, such as the T5 encoders' fp32 option) run the fp32
 matrix-core GEMM, in fp32 throughout as F.linear does. A K or N off the kernel's multiples (64
 and 4 for bf16, 4 and 4 for fp32) is zero-padded once on the weight (and per call on the input).
@@ -78,7 +79,8 @@ class _RocmLinearBase(nn.Module):
             return x.new_empty(*shape[:-1], self.out_features)
         # a few rows run on the GEMV kernel with the weight as is; the GEMM reads the weight
         # zero-padded to its tile multiples (built once, only for odd shapes)
-        wg = w.detach() if library._gemv_fits(m, self.in_features) else self._weight_for_gemm()[0]
+        wg = w.detach() if library._gemv_fits(
+            m, self.in_features, self.out_features) else self._weight_for_gemm()[0]
         y = library.linear(x2, wg, b, self.out_features)
         return y.reshape(*shape[:-1], self.out_features).to(x.dtype)
 

@@ -735,37 +735,78 @@ __global__ __launch_bounds__(256) void gate_residual_kernel(
 // the input dtype first, as the reference's `silu(emb)` tensor is). W is read once, 16 bytes
 // per lane per step, so the kernel runs at HBM speed. M is a compile-time bound on the rows;
 // rows m..M-1 of the LDS stage are zero and never stored.
-template <typename T, int M>
+//
+// A slice of x read from LDS (fp32, twice W's bytes) serves the CP columns of a wave, so CP = 4
+// where that leaves enough waves (n >= 8192) and 2 below; a group is three 512-wide slices,
+// unguarded, CP x 3 loads of 1 KB in flight. A workgroup lives for one or two groups, so its start
+// counts too: up to 16 input values per thread go to registers first, then the first group of W is
+// requested, and only then are the inputs staged, behind those loads (loads return in order:
+// inputs requested after W would wait for it). 1 x 3072 x 18432 (113 MB) 29.7 -> 24.2 us, 26.0 with
+// two columns of six slices; 1 x 3072 x 264192 244 -> 238 us (6.8 TB/s).
+template <typename T, int M, int CP>
 __global__ __launch_bounds__(256) void gemv_kernel(const T* __restrict__ x, int m, int k,
                                                    int64_t ldx, const bf16* __restrict__ w,
                                                    int64_t ldw, int64_t n,
                                                    const T* __restrict__ bias,
                                                    T* __restrict__ y, int64_t ldy, int act) {
   extern __shared__ float xs[];  // [M][k]
-  for (int i = threadIdx.x; i < M * k; i += 256) {
-    const int r = i / k, kk = i - r * k;
-    float v = 0.f;
-    if (r < m) {
-      v = Elt<T>::load(x + r * ldx + kk);
-      if (act == 1) {
-        T t;
-        Elt<T>::store(&t, silu(v));
-        v = Elt<T>::load(&t);
-      }
-    }
-    xs[i] = v;
-  }
-  __syncthreads();
   const int lane = threadIdx.x & 63;
-  // Two columns per wave and 3072-wide groups of six 1 KB loads per column, unguarded: twelve
-  // loads in flight per wave before the first multiply; the k % 3072 tail is guarded.
-  constexpr int U = 6, CP = 2;
+  constexpr int U = 3;  // the k % 1536 tail is guarded
   const int kfull = k - k % (U * 512);
   const int64_t step = (int64_t)gridDim.x * 4 * CP;
-  for (int64_t c0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * CP; c0 < n; c0 += step) {
-    const bf16* wr[CP];
+  // wave-uniform, so that a row is a scalar base and the lane an offset
+  const int64_t first =
+      ((int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * CP;
+  const bf16* wr[CP];
+  u32x4 wv[CP][U];
+  auto rows_at = [&](int64_t c0) {
 #pragma unroll
-    for (int p = 0; p < CP; ++p) wr[p] = w + (c0 + p < n ? c0 + p : n - 1) * ldw + lane * 8;
+    for (int p = 0; p < CP; ++p) wr[p] = w + (c0 + p < n ? c0 + p : n - 1) * ldw;
+  };
+  auto load_group = [&](int g) {
+#pragma unroll
+    for (int p = 0; p < CP; ++p)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        wv[p][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr[p] + g + u * 512 + lane * 8));
+  };
+  auto input = [&](int i) {  // x value i of [M][k], zero past the rows
+    const int r = i / k;
+    return r < m ? Elt<T>::load(x + r * ldx + (i - r * k)) : 0.f;
+  };
+  auto stage = [&](int i, float v) {
+    if (act == 1) {
+      T t;
+      Elt<T>::store(&t, silu(v));
+      v = Elt<T>::load(&t);
+    }
+    xs[i] = v;
+  };
+  constexpr int XR = 16;
+  const int nx = M * k;
+  rows_at(first);
+  if (nx <= XR * 256) {
+    float xv[XR];
+#pragma unroll
+    for (int u = 0; u < XR; ++u) {
+      const int i = threadIdx.x + 256 * u;
+      xv[u] = i < nx ? input(i) : 0.f;
+    }
+    if (kfull > 0) load_group(0);  // past the last column: its rows are clamped to column n - 1
+#pragma unroll
+    for (int u = 0; u < XR; ++u) {
+      const int i = threadIdx.x + 256 * u;
+      if (i < nx) stage(i, xv[u]);
+    }
+  } else {
+    for (int i = threadIdx.x; i < nx; i += 256) stage(i, input(i));
+    if (kfull > 0) load_group(0);
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's stores; W's loads stay in flight
+  asm volatile("s_barrier" ::: "memory");
+  bool loaded = kfull > 0;  // the first group of this wave's first columns
+  for (int64_t c0 = first; c0 < n; c0 += step) {
+    rows_at(c0);
     float acc[CP][M];
 #pragma unroll
     for (int p = 0; p < CP; ++p)
@@ -782,21 +823,20 @@ __global__ __launch_bounds__(256) void gemv_kernel(const T* __restrict__ x, int 
       }
     };
     for (int g = 0; g < kfull; g += U * 512) {
-      u32x4 wv[CP][U];
+      if (!loaded) load_group(g);
+      loaded = false;
 #pragma unroll
-      for (int p = 0; p < CP; ++p)
+      for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          wv[p][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr[p] + g + u * 512));
-#pragma unroll
-      for (int p = 0; p < CP; ++p)
-#pragma unroll
-        for (int u = 0; u < U; ++u) fma8(wv[p][u], g + u * 512 + lane * 8, acc[p]);
+        for (int p = 0; p < CP; ++p) fma8(wv[p][u], g + u * 512 + lane * 8, acc[p]);
+        // one slice's inputs at a time: read ahead, they took the registers of half the waves
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     for (int c = kfull; c + lane * 8 < k; c += 512) {
 #pragma unroll
       for (int p = 0; p < CP; ++p)
-        fma8(*reinterpret_cast<const u32x4*>(wr[p] + c), c + lane * 8, acc[p]);
+        fma8(*reinterpret_cast<const u32x4*>(wr[p] + c + lane * 8), c + lane * 8, acc[p]);
     }
 #pragma unroll
     for (int p = 0; p < CP; ++p) {
@@ -1280,13 +1320,19 @@ template <typename T>
 static int launch_gemv(const void* x, int64_t m, int mb, int64_t k, int64_t ldx, const void* w,
                        int64_t ldw, int64_t n, const void* bias, void* y, int64_t ldy, int act,
                        hipStream_t s) {
-  int64_t blocks = (n + 7) / 8;
+  const int64_t cols = n >= 8192 ? 16 : 8;  // per workgroup
+  int64_t blocks = (n + cols - 1) / cols;
   if (blocks > 8192) blocks = 8192;
   const size_t lds = (size_t)(mb * k * 4);
-#define DLT_GEMV(M)                                                                          \
-  hipLaunchKernelGGL((gemv_kernel<T, M>), dim3((unsigned)blocks), dim3(256), lds, s,         \
-                     (const T*)x, (int)m, (int)k, ldx, (const bf16*)w, ldw, n, (const T*)bias,     \
-                     (T*)y, ldy, act)
+#define DLT_GEMV_CP(M, CP)                                                                  \
+  hipLaunchKernelGGL((gemv_kernel<T, M, CP>), dim3((unsigned)blocks), dim3(256), lds, s,    \
+                     (const T*)x, (int)m, (int)k, ldx, (const bf16*)w, ldw, n,              \
+                     (const T*)bias, (T*)y, ldy, act)
+#define DLT_GEMV(M)                       \
+  do {                                    \
+    if (cols == 16) DLT_GEMV_CP(M, 4);    \
+    else DLT_GEMV_CP(M, 2);               \
+  } while (0)
   switch (mb) {
     case 1: DLT_GEMV(1); break;
     case 2: DLT_GEMV(2); break;
@@ -1294,6 +1340,7 @@ static int launch_gemv(const void* x, int64_t m, int mb, int64_t k, int64_t ldx,
     default: DLT_GEMV(8); break;
   }
 #undef DLT_GEMV
+#undef DLT_GEMV_CP
   return dlt_check_launch("gemv");
 }
 
