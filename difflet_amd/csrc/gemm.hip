@@ -102,8 +102,12 @@ __host__ __device__ inline int sk_slot(const SkPlan& p, int c, int r, int gi) {
 constexpr int64_t SK_CTR_BYTES = 16384;        // one int counter per split tile
 constexpr int SK_MAX_TILES = (int)(SK_CTR_BYTES / 4);
 constexpr int64_t SK_SLOT_BYTES = 256 * 256 * 4;  // fp32 accumulators of one 256 x 256 tile
-constexpr int SK_MIN_STAGES = 8;               // shortest K range worth a workgroup
+constexpr int SK_MIN_STAGES = 6;               // shortest K range worth a workgroup
 constexpr int SK_MIN_SAVED_STAGES = 24;         // shortest cut off the busiest K walk (below)
+
+constexpr int SK_MIN_SAVED_OWN = 40;            // the same on scratch of the launch's own
+constexpr int SK_SAVED_ANYWAY = 48;             // a cut worth its partial sums in any launch
+constexpr int64_t SMALL_SCRATCH_CAP = 64LL << 20;  // fp32 sums of a small launch's K pieces
 
 struct GemmArgs {
   GemmProblemDev p[MAX_PROBLEMS];
@@ -1032,8 +1036,13 @@ static int64_t sk_workspace_bytes(int groups) {
 // launches (FF2 MXFP8 365 -> 316 us, bf16 576 -> 483 us; 60 and 30 stages saved) and Wan's
 // 80-tile bf16 text k/v projection (93 -> 87 us, 40 saved), and loses on FLUX's 216-, 648-
 // and 864-tile ones (out projection bf16 87 -> 101 us, FF1 fp8 169 -> 198 us) and on the MXFP8
-// twin of that k/v projection (49 -> 66 us, 20 saved), which these rules leave whole.
-static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes) {
+// twin of that k/v projection (49 -> 66 us, 20 saved), which these rules leave whole. In a long
+// launch a quarter is more than it takes: SK_SAVED_ANYWAY stages saved pay whatever they are a part
+// of (5120 x 5120 over 14000 rows, 1100 tiles, 50 saved: 656 -> 606 us; at 42 saved, 3072 x 12288,
+// 1296 tiles ran 467 -> 461 and 1056 tiles 394 -> 402). A launch on scratch of its own (`own`) also
+// clears the counters and asks for SK_MIN_SAVED_OWN: 324 tiles at K = 3072, 30 saved, took 158 us
+// split and 151 whole; 264 tiles there, 42 saved, 150 whole and 131 split; at K = 12288 531 and 369.
+static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes, bool own = false) {
   const int nu = (nk + gran - 1) / gran;
   SkPlan pl = {T, 0, nu, gran, 0, 0, 0, 0};
   constexpr int NX = 8;
@@ -1046,7 +1055,8 @@ static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes) {
   const int64_t span = (units + NX - 1) / NX;
   if (S > SK_MAX_TILES || ws_bytes < sk_workspace_bytes(cus) ||
       units / NX < std::max(1, SK_MIN_STAGES / gran) ||
-      4 * (nu - span) < (int64_t)waves * nu || (nu - span) * gran < SK_MIN_SAVED_STAGES)
+      (nu - span) * gran < (own ? SK_MIN_SAVED_OWN : SK_MIN_SAVED_STAGES) ||
+      (4 * (nu - span) < (int64_t)waves * nu && (nu - span) * gran < SK_SAVED_ANYWAY))
     return pl;
   pl.dp = dp;
   pl.groups = cus;
@@ -1081,11 +1091,19 @@ static SmallPlan small_plan_of(int64_t m, int64_t n, int64_t k, int64_t scratch,
   return small_plan(small_elem<E>(), m, n, k, cus, scratch, us);
 }
 
+// Counters of the split schedule to zero before a launch on scratch nobody zeroed (a kernel, not
+// a memset: the pair can be captured into a graph).
+__global__ void gemm_zero_counters(int* __restrict__ ctr, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) ctr[i] = 0;
+}
+
+// own_scratch: the workspace is this launch's alone (difflet_rocm_gemm_scratch_bytes), not zeroed.
 template <Elem E>
 static int gemm_launch(const char* name, int nproblems, const difflet_gemm_problem* problems,
                        int64_t n, int64_t k, int epilogue, int64_t act_col_start,
                        void* workspace, int64_t workspace_bytes, const difflet_gemm_qk* qk,
-                       hipStream_t stream) {
+                       hipStream_t stream, bool own_scratch = false) {
   constexpr int KT = ElemTraits<E>::KT;
   constexpr int EB = ElemTraits<E>::BYTES;
   DLT_REQUIRE(problems && nproblems >= 1 && nproblems <= MAX_PROBLEMS, DIFFLET_EINVAL,
@@ -1221,13 +1239,14 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
     args.rope_sin = qk->sin;
   }
   args.sk = sk_plan((int)tiles, (int)(k / KT), E == Elem::MX ? 4 : 1,
-                    workspace ? gemm_device_cus() : 0, workspace ? workspace_bytes : 0);
+                    workspace ? gemm_device_cus() : 0, workspace ? workspace_bytes : 0,
+                    own_scratch);
   // launches of few tiles: smaller tiles, K cut into pieces (gemm_small.hip)
   if (nproblems == 1 && !qk &&
       (epilogue == DIFFLET_EPI_NONE || epilogue == DIFFLET_EPI_GATE_RESIDUAL)) {
-    const SmallPlan plan =
-        small_plan_of<E>(problems[0].m, n, k, workspace ? workspace_bytes - SK_CTR_BYTES : 0,
-                         args.sk);
+    const int64_t bytes = workspace ? workspace_bytes - SK_CTR_BYTES : 0;
+    const SmallPlan plan = small_plan_of<E>(
+        problems[0].m, n, k, own_scratch ? std::min(bytes, SMALL_SCRATCH_CAP) : bytes, args.sk);
     if (plan.bm > 0) {
       gemm_small(small_elem<E>(), plan, problems[0], n, k, epilogue == DIFFLET_EPI_GATE_RESIDUAL,
                  args.p[0].rows_per_batch, workspace ? (uint8_t*)workspace + SK_CTR_BYTES : nullptr,
@@ -1239,6 +1258,12 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
   constexpr int NT = ElemTraits<E>::WN;
   dim3 grid((unsigned)(args.sk.dp + args.sk.groups)), block(128 * NT);
   const bool split = args.sk.groups > 0;
+  if (split && own_scratch) {
+    hipLaunchKernelGGL(gemm_zero_counters, dim3((unsigned)((args.sk.S + 255) / 256)), dim3(256), 0,
+                       stream, reinterpret_cast<int*>(workspace), args.sk.S);
+    const int st = dlt_check_launch(name);
+    if (st != DIFFLET_OK) return st;
+  }
   auto go = [&](auto epi, auto fused) {
     constexpr int EP = decltype(epi)::value;
     constexpr bool Q = decltype(fused)::value;
@@ -1288,13 +1313,19 @@ extern "C" int64_t difflet_rocm_gemm_workspace_bytes(void) {
 extern "C" int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m >= (1LL << 30) || n >= (1LL << 30) || k >= (1LL << 30))
     return 0;
-  constexpr int64_t cap = 64LL << 20;
-  const SkPlan whole = {};
-  const SmallPlan p = kind == 0   ? small_plan_of<Elem::BF16>(m, n, k, cap, whole)
-                      : kind == 1 ? small_plan_of<Elem::FP8>(m, n, k, cap, whole)
-                      : kind == 2 ? small_plan_of<Elem::MX>(m, n, k, cap, whole)
-                                  : small_plan(SmallElem::F32, m, n, k, gemm_device_cus(), cap, 2e30);
-  return p.pieces > 1 ? SK_CTR_BYTES + p.pieces * m * n * 4 : 0;
+  constexpr int64_t cap = SMALL_SCRATCH_CAP;
+  const int cus = gemm_device_cus();
+  const int64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
+  SkPlan sk = {};
+  if (kind < 3 && tiles < (1LL << 30))
+    sk = sk_plan((int)tiles, (int)(k / (kind == 0 ? 64 : 128)), kind == 2 ? 4 : 1, cus, INT64_MAX,
+                 true);
+  const SmallPlan p = kind == 0   ? small_plan_of<Elem::BF16>(m, n, k, cap, sk)
+                      : kind == 1 ? small_plan_of<Elem::FP8>(m, n, k, cap, sk)
+                      : kind == 2 ? small_plan_of<Elem::MX>(m, n, k, cap, sk)
+                                  : small_plan(SmallElem::F32, m, n, k, cus, cap, 2e30);
+  if (p.bm > 0) return p.pieces > 1 ? SK_CTR_BYTES + p.pieces * m * n * 4 : 0;
+  return sk.groups > 0 ? sk_workspace_bytes(cus) : 0;
 }
 
 extern "C" int difflet_rocm_gemm_single(int kind, const void* a, int64_t lda, const void* w,
@@ -1315,10 +1346,14 @@ extern "C" int difflet_rocm_gemm_single(int kind, const void* a, int64_t lda, co
   q.m = m;
   q.rows_per_batch = m;
   DLT_REQUIRE(kind >= 0 && kind <= 2, DIFFLET_EINVAL, "gemm_single: unknown kind %d", kind);
-  auto* fn = kind == 0   ? difflet_rocm_gemm_bf16
-             : kind == 1 ? difflet_rocm_gemm_fp8_rowwise
-                         : difflet_rocm_gemm_mxfp8;
-  return fn(1, &q, n, k, DIFFLET_EPI_NONE, 0, workspace, workspace_bytes, nullptr, stream);
+  auto run = [&](auto e, const char* name) {
+    return gemm_launch<decltype(e)::value>(name, 1, &q, n, k, DIFFLET_EPI_NONE, 0, workspace,
+                                           workspace_bytes, nullptr, (hipStream_t)stream, true);
+  };
+  using std::integral_constant;
+  if (kind == 0) return run(integral_constant<Elem, Elem::BF16>{}, "gemm_bf16");
+  if (kind == 1) return run(integral_constant<Elem, Elem::FP8>{}, "gemm_fp8_rowwise");
+  return run(integral_constant<Elem, Elem::MX>{}, "gemm_mxfp8");
 }
 
 extern "C" int difflet_rocm_gemm_bf16(int nproblems, const difflet_gemm_problem* problems,

@@ -258,6 +258,7 @@ class QkNormRope:
 
 _GEMM_FN = {"bf16": "difflet_rocm_gemm_bf16", "fp8": "difflet_rocm_gemm_fp8_rowwise",
             "mx": "difflet_rocm_gemm_mxfp8"}
+_COUNTER_BYTES = 16384  # the split schedule's counters, at the front of a GEMM workspace
 _KIND_ID = {"bf16": 0, "fp8": 1, "mx": 2, "f32": 3}
 
 
@@ -447,8 +448,10 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
             if len(problems) == 1 and qk is None and epilogue in (_lib.EPI_NONE,
                                                                   _lib.EPI_GATE_RESIDUAL):
                 nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID[kind], arr[0].m, n, k)
+                # a buffer large enough for the split schedule needs its counters zeroed here
                 if nbytes:
                     workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+                    workspace[:_COUNTER_BYTES].zero_()
         else:
             raise ValueError("workspace must be 'shared', 'call', a tensor or None, "
                              f"got {workspace!r}")

@@ -219,14 +219,13 @@ typedef struct difflet_gemm_qk {
  * as whole tiles and cuts the last wave's tiles along K over the 8 XCDs: in groups of 32 tiles,
  * each XCD takes a contiguous range of (group, K unit) pairs and its 32 workgroups walk the
  * same K units of 32 neighbouring tiles together (whole-tile L2 sharing is kept). The cut is
- * made only when it takes a quarter and at least 24 K stages off the launch's K walk
+ * made only when it takes a quarter and at least 24 K stages, or 48, off the launch's K walk
  * (Qwen-Image's 336-tile projections qualify; FLUX's 216-tile ones, which would save an
  * eighth, stay whole, and so does an MXFP8 projection of 512 rows at K = 4096). The workgroup
  * finishing a cut tile adds the fp32 partial sums of the others in a fixed order, so results
  * are deterministic for a given device. With workspace NULL (or too small) every tile runs
  * whole on one workgroup. A launch of one problem with few tiles (up to 4096 rows, epilogue NONE
- * or GATE_RESIDUAL, no fused q/k norm) runs in smaller tiles instead, and with a workspace of
- * difflet_rocm_gemm_scratch_bytes or more may cut K into pieces, whose fp32 sums a second kernel
+ * or GATE_RESIDUAL, no fused q/k norm) runs in smaller tiles instead, and with a workspace may cut K into pieces, whose fp32 sums a second kernel
  * adds in order (nothing in the workspace need be zero for that, and its counters stay as they
  * are). The workspace must be zero-filled once when allocated; the GEMMs
  * leave it zeroed. Launches that may overlap in time (different streams) must not share one.
@@ -237,13 +236,14 @@ int64_t difflet_rocm_gemm_workspace_bytes(void);
 
 /* Bytes of scratch with which one m x n x k problem (kind 0 bf16, 1 fp8 per row, 2 MXFP8, 3
  * fp32; epilogue NONE or GATE_RESIDUAL) runs at its fastest among the small-launch plans: passed as the
- * workspace, not zeroed, used by that launch only. 0: no scratch helps. Always less than
- * difflet_rocm_gemm_workspace_bytes, so such a buffer never serves the split schedule, which
- * needs zeroed counters. */
+ * workspace of difflet_rocm_gemm_single or difflet_rocm_gemm_f32_scratch, not zeroed, used by that
+ * launch only. 0: no scratch helps. */
 int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k);
 
 /* One problem with EPI_NONE through the GEMM of `kind` (0 bf16, 1 fp8 per row, 2 MXFP8), its
- * operands as plain arguments. */
+ * operands as plain arguments. The workspace is scratch of this launch alone
+ * (difflet_rocm_gemm_scratch_bytes, or NULL): a launch that cuts its last wave of tiles clears the
+ * counters it uses first. */
 int difflet_rocm_gemm_single(int kind, const void* a, int64_t lda, const void* w, int64_t ldw,
                              void* c, int64_t ldc, const void* bias, const void* a_scale,
                              const void* w_scale, int64_t m, int64_t n, int64_t k,

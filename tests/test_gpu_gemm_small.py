@@ -92,3 +92,29 @@ def test_fp32_gemm(gpu, m, n, k):
         y = r.to(gpu)
         kernels.gemm_f32(ag, wg, b.to(gpu), residual=y, out=y, workspace=workspace)
         assert ((y.double().cpu() - ref - r.double()).norm() / ref.norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "mx"])
+@pytest.mark.parametrize("m,n,k", [(6889, 3072, 6144), (6700, 12288, 10240)])
+def test_linear_call_split_schedule_on_scratch(gpu, kind, m, n, k):
+    """A last wave of tiles cut over the XCDs on scratch of the call, which nobody zeroed: equal on
+    reruns over garbage, and to whole tiles within fp32 summation order (2e-3, a bf16 step)."""
+    if kind != "bf16":
+        k *= 2  # the same number of K stages
+    print(f"split on scratch {kind} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m)
+    a = torch.randn(m, k, generator=g, device=gpu).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=gpu) * 0.05).bfloat16()
+    aq, wq, sa, sw = _operands(kind, a, w, gpu)
+    kid = {"bf16": 0, "fp8": 1, "mx": 2}[kind]
+    nbytes = _lib.load().difflet_rocm_gemm_scratch_bytes(kid, m, n, k)
+    assert nbytes == _lib.load().difflet_rocm_gemm_workspace_bytes()  # the split schedule's
+    outs = []
+    for _ in range(2):
+        torch.full((nbytes,), 0xff, dtype=torch.uint8, device=gpu)  # freed: the scratch's garbage
+        outs.append(kernels.gemm_call(kind, aq, wq, None, sa, sw))
+    assert torch.equal(outs[0], outs[1])
+    whole = torch.empty_like(outs[0])
+    kernels.gemm_grouped([kernels.Problem(aq, wq, whole, a_scale=sa, w_scale=sw)], kind=kind)
+    d = (outs[0].float() - whole.float()).norm() / whole.float().norm()
+    assert d.item() < 2e-3
