@@ -548,7 +548,7 @@ __device__ __forceinline__ void vm_phase_barrier() {
 // Masked keys take a raw score of -2^126 / 2^e (2^e <= the scale, at least 1): a power of two,
 // so its product with the scale is exact and finite and a fully masked row's exponentials are
 // all exp2(0): the row averages v. 24 x 6889 queries x 7145 keys: 1473 us for the joint call on
-// the single-group masked kernel, with the copies and the bounds' fills; 558 us here. The
+// the single-group masked kernel, with the copies and the bounds' fills; 603 us here. The
 // plain instance (GEN false) is compiled apart and keeps its registers.
 template <typename T, bool GEN>
 __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
@@ -815,23 +815,44 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
         }
       return ls;
     };
-    float ls = exps(m_run);
-    if (__any(!(ls < MfmaT<T>::kLazyLimit))) {
-      float mx = -INFINITY;
+    float ls;
+    if constexpr (GEN) {
+      // the reference is the running max itself, moved whenever a score passes it: a row's largest
+      // probability is then exactly 1, free of the 16-bit rounding, as in the single-group kernel
+      // that these calls ran on (relative to an older max their error is 2 to 6 % larger)
+      float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
-      for (int kt2 = 0; kt2 < 2; ++kt2)
+      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, fmaxf(s[0][v], s[1][v]));
+      if (__any(!(mx * cmul <= m_run))) {
+        const float m_new = fmaxf(m_run, pair_max(mx) * cmul);
+        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[kt2][v]);
-      mx = pair_max(mx);
-      const float m_new = fmaxf(m_run, mx * cmul);
-      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-      m_run = m_new;
-      l_run *= alpha;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][v] *= alpha;
+          for (int v = 0; v < 16; ++v) acc[i][v] *= alpha;
+      }
       ls = exps(m_run == -INFINITY ? 0.f : m_run);
+    } else {
+      ls = exps(m_run);
+      if (__any(!(ls < MfmaT<T>::kLazyLimit))) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[kt2][v]);
+        mx = pair_max(mx);
+        const float m_new = fmaxf(m_run, mx * cmul);
+        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][v] *= alpha;
+        ls = exps(m_run == -INFINITY ? 0.f : m_run);
+      }
     }
     l_run += ls;
     // P is computed here, in the softmax phase: without the pins the compiler sinks the
