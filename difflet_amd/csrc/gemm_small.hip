@@ -432,7 +432,7 @@ __global__ __launch_bounds__(256) void gemm_small_reduce(const SmallArgs args) {
 //    or more workgroups at a time, kStageF32 each with one, two or more of them on the unit
 //    (matrix-core time 0.43 and 1.74 at 2.35 GHz);
 //  - cutting K adds the reduce launch and the sums' trip out and back at about 5 TB/s.
-// 16 and 8 rows apart from the boundary the choices measured (bf16, K = N = 3072 / 12288 x 3072 /
+// What the choices measured (bf16, 3072 x 3072 / 12288 x 3072 /
 // 5120 x 5120, 256 x 256 tiles -> the plan's): 64 rows 57 -> 16, 65 -> 23, 50 -> 18; 512 rows
 // 62 -> 19, 77 -> 55, 74 -> 44; 1024 rows 66 -> 27, 114 -> 97, 94 -> 75; fp8 12288 x 3072 at 16,
 // 512 and 1024 rows 51 -> 18, 60 -> 32, 78 -> 46. Past 4096 rows the 256 x 256 tiles fill the
@@ -444,7 +444,6 @@ SmallPlan small_plan(SmallElem e, int64_t m, int64_t n, int64_t k, int cus, int6
   if (cus <= 0 || m <= 0 || (m > 4096 && !f32)) return best;
   const int eb = f32 ? 4 : e == SmallElem::BF16 ? 2 : 1;
   const int nk = (int)((k * eb + 127) / 128), gran = e == SmallElem::MX ? 4 : 1;
-  // PLAN
   static const int kRows[3] = {64, 128, 256};
   static const double kStage[3][3] = {{0.36, 0.52, 0.90}, {0.30, 0.43, 0.88}, {0.38, 0.60, 0.90}};
   static const double kStageF32[2][3] = {{0.62, 0.53, 0.505}, {2.05, 1.95, 1.93}};
