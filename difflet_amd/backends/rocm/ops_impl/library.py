@@ -10,8 +10,9 @@ difflet/backends/tpu/ops_impl/collectives.py:99-150).
 A custom_op's Python layers cost about 10 us a call, as much as a short linear on the device. So
 the operators of the linears and the attention each have a twin, ``<name>_infer``, with the same
 implementation and fake but a bare dispatcher registration; the functions here call the twin for
-device tensors that need no gradient, outside torch.compile. Everything else (graphs, inputs that
-require grad, whose backward custom_op refuses, host tensors) goes to the custom_op.
+device tensors that need no gradient, in plain eager execution (_eager). Everything else (compiled
+and recorded graphs, functorch transforms, inputs that require grad, whose backward custom_op
+refuses, host tensors) goes to the custom_op. The twin's own backward refuses too.
 
 Every operator is functional: it allocates and returns a new contiguous tensor and mutates no
 argument. Shape and dtype checks that raise for unsupported inputs stay in the op modules, so
@@ -33,12 +34,18 @@ _INFER = torch.library.Library("difflet_rocm", "FRAGMENT")  # noqa: TOR901
 
 
 def _infer_twin(op, impl, fake):
-    """The operator <op's name>_infer of op's signature: impl on the device, fake for tracing."""
+    """The operator <op's name>_infer of op's signature: impl on the device, fake for tracing, and
+    as the custom_op no formula for the backward."""
     schema = op._opoverload._schema
     name = schema.name.split("::")[1]
     _INFER.define(str(schema).split("::")[1].replace(f"{name}(", f"{name}_infer(", 1))
     _INFER.impl(f"{name}_infer", impl, "CUDA")
     torch.library.register_fake(f"difflet_rocm::{name}_infer", fake, lib=_INFER)
+
+    def no_backward(ctx, *grads):
+        raise RuntimeError(f"difflet_rocm::{name} has no backward: it runs inference only")
+
+    torch.library.register_autograd(f"difflet_rocm::{name}_infer", no_backward, lib=_INFER)
     return getattr(torch.ops.difflet_rocm, f"{name}_infer").default
 
 
@@ -49,6 +56,35 @@ def _plain(*tensors: Optional[Tensor]) -> bool:
         if t is not None and (not t.is_cuda or (grad and t.requires_grad)):
             return False
     return True
+
+
+_functorch_level = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_pre_dispatch_modes = torch._ops._len_torch_dispatch_stack_pre_dispatch
+_jit_trace = torch._C._get_tracing_state
+_forward_ad = torch.autograd.forward_ad
+_below_autograd = torch._C._AutoDispatchBelowAutograd
+_SCALARS = frozenset((type(None), int, float, bool))
+_ARGUMENTS = _SCALARS | {Tensor, torch.nn.Parameter}
+
+
+def _eager() -> bool:
+    """Nothing records, transforms or differentiates the calls: no torch.compile, jit or dispatch
+    mode (make_fx, fake tensors), no functorch level (a batched tensor denies the gradient that
+    the tensor under it needs), no forward-mode level."""
+    return not (torch.compiler.is_compiling() or _functorch_level() is not None
+                or _dispatch_modes() or _pre_dispatch_modes() or _jit_trace() is not None
+                or _forward_ad._current_level >= 0)
+
+
+def _infer(op, twin, *args):
+    """twin(*args) where it can stand in for op, else op(*args). The twin runs below autograd, as
+    custom_op's implementations do: its kernel there is only for calls that come another way."""
+    if (_eager() and _ARGUMENTS.issuperset(map(type, args))  # no tensor subclass
+            and _plain(*[a for a in args if type(a) not in _SCALARS])):
+        with _below_autograd():
+            return twin(*args)
+    return op(*args)
 
 
 # ---------------------------------------------------------------------------------- attention
@@ -72,9 +108,8 @@ _attention_infer = _infer_twin(_attention_op, _attention_impl, _attention_fake)
 def attention(q: Tensor, k: Tensor, v: Tensor, scale: float, causal: bool,
               attention_mask: Optional[Tensor], bound_min: Optional[Tensor],
               bound_max: Optional[Tensor]) -> Tensor:
-    if not torch.compiler.is_compiling() and _plain(q, k, v, attention_mask, bound_min, bound_max):
-        return _attention_infer(q, k, v, scale, causal, attention_mask, bound_min, bound_max)
-    return _attention_op(q, k, v, scale, causal, attention_mask, bound_min, bound_max)
+    return _infer(_attention_op, _attention_infer, q, k, v, scale, causal, attention_mask,
+                  bound_min, bound_max)
 
 
 def _attention_joint_impl(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
@@ -98,9 +133,8 @@ _attention_joint_infer = _infer_twin(_attention_joint_op, _attention_joint_impl,
 
 def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
                     key_count: Optional[Tensor], count_offset: int) -> Tensor:
-    if not torch.compiler.is_compiling() and _plain(q, k, v, k2, v2, key_count):
-        return _attention_joint_infer(q, k, v, k2, v2, scale, key_count, count_offset)
-    return _attention_joint_op(q, k, v, k2, v2, scale, key_count, count_offset)
+    return _infer(_attention_joint_op, _attention_joint_infer, q, k, v, k2, v2, scale, key_count,
+                  count_offset)
 
 
 # ------------------------------------------------------------------------------------- linear
@@ -143,9 +177,7 @@ _linear_infer = _infer_twin(_linear_op, _linear_impl, _linear_fake)
 
 
 def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
-    if not torch.compiler.is_compiling() and _plain(x, w, bias):
-        return _linear_infer(x, w, bias, out_features)
-    return _linear_op(x, w, bias, out_features)
+    return _infer(_linear_op, _linear_infer, x, w, bias, out_features)
 
 
 def _linear_f32_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
@@ -175,9 +207,7 @@ _linear_f32_infer = _infer_twin(_linear_f32_op, _linear_f32_impl, _linear_f32_fa
 
 
 def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
-    if not torch.compiler.is_compiling() and _plain(x, w, bias):
-        return _linear_f32_infer(x, w, bias, out_features)
-    return _linear_f32_op(x, w, bias, out_features)
+    return _infer(_linear_f32_op, _linear_f32_infer, x, w, bias, out_features)
 
 
 def _fp8_linear_impl(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
@@ -203,9 +233,7 @@ _fp8_linear_infer = _infer_twin(_fp8_linear_op, _fp8_linear_impl, _fp8_linear_fa
 
 def fp8_linear(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
                mx: bool) -> Tensor:
-    if not torch.compiler.is_compiling() and _plain(x, w_kernel, w_scale, bias):
-        return _fp8_linear_infer(x, w_kernel, w_scale, bias, mx)
-    return _fp8_linear_op(x, w_kernel, w_scale, bias, mx)
+    return _infer(_fp8_linear_op, _fp8_linear_infer, x, w_kernel, w_scale, bias, mx)
 
 
 # ---------------------------------------------------------------------------- norms, rotary

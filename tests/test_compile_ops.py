@@ -103,3 +103,67 @@ def test_infer_twins_mirror_the_custom_ops():
         assert y.shape == (33, 99) and y.requires_grad
         y = library.linear(x, w.detach(), None, 99)
         assert y.shape == (33, 99) and y.dtype == torch.bfloat16 and y.is_cuda
+
+
+def _linear_args():
+    bf = dict(dtype=torch.bfloat16, device="cuda")
+    return torch.empty(5, 33, 384, **bf), torch.empty(100, 384, **bf)
+
+
+def _grad_nodes(y):
+    seen, todo = set(), [y.grad_fn]
+    while todo:
+        node = todo.pop()
+        if node is not None and node not in seen:
+            seen.add(node)
+            todo += [n for n, _ in node.next_functions]
+    return {n.name() for n in seen}
+
+
+@pytest.mark.parametrize("batched", [False, True])
+@pytest.mark.parametrize("call", ["linear", "linear_infer"])
+def test_gradients_are_refused_also_under_vmap(call, batched):
+    """Inputs that need a gradient get the node whose backward raises, whether the call comes through
+    library.linear or names the twin, and where vmap's batched tensor hides the gradient."""
+    with FakeTensorMode():
+        x, w = _linear_args()
+        x.requires_grad_()
+        fn = library.linear if call == "linear" else torch.ops.difflet_rocm.linear_infer
+        f = lambda r: fn(r, w, None, 100)  # noqa: E731
+        names = _grad_nodes(torch.vmap(f)(x) if batched else f(x[0]))
+    assert any(n.startswith("GeneratedBackwardFor_difflet_rocm_linear") for n in names), names
+    assert not any("NotImplemented" in n for n in names), names
+
+
+@pytest.mark.parametrize("pre_dispatch", [False, True])
+def test_recorded_graphs_hold_the_custom_op(pre_dispatch):
+    """A graph recorded with inputs that need no gradient may be replayed with ones that do."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    with FakeTensorMode():
+        x, w = _linear_args()
+        gm = make_fx(lambda a: library.linear(a, w, None, 100), pre_dispatch=pre_dispatch)(x[0])
+    calls = [n.target for n in gm.graph.nodes if n.op == "call_function"]
+    assert torch.ops.difflet_rocm.linear.default in calls
+    assert torch.ops.difflet_rocm.linear_infer.default not in calls
+
+
+def test_twins_are_for_plain_eager_execution_only():
+    import torch.autograd.forward_ad as fwd
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        pass
+
+    assert library._eager()
+    with Mode():
+        assert not library._eager()
+    with fwd.dual_level():
+        assert not library._eager()
+    seen = []
+    torch.vmap(lambda t: (seen.append(library._eager()), t)[1])(torch.zeros(2))
+    torch.func.grad(lambda t: (seen.append(library._eager()), t.sum())[1])(torch.zeros(2))
+    torch.jit.trace(lambda t: (seen.append(library._eager()), t + 1)[1], torch.zeros(2),
+                    check_trace=False)
+    assert seen == [False, False, False]
+    assert library._eager()

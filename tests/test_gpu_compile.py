@@ -234,3 +234,19 @@ def test_compiled_flux_single_block_matches_the_oracle(gpu, kind, parity):
     parity("compiled op-module single block fp8, rel L2 vs same-law oracle", e, 3e-2)
     assert e < 3e-2
     assert abs(fmt_dev - fmt_ref) < 0.1 * fmt_ref
+
+
+def test_gradients_through_the_kernels_are_refused(gpu):
+    """The operators run inference only: a backward through one raises, under vmap and functorch too,
+    instead of leaving the gradient out. Without gradients vmap gives each row's own result."""
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(3, 16, D, generator=g).bfloat16().to(gpu)
+    lin = ColumnParallelLinear(D, D, dtype=torch.bfloat16, device=gpu).requires_grad_(False)
+    assert torch.equal(torch.vmap(lin)(x), torch.stack([lin(r) for r in x]))
+    leaf = x.clone().requires_grad_()
+    for y in (lin(leaf), torch.vmap(lin)(leaf)):
+        with pytest.raises(RuntimeError):
+            y.sum().backward()
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda a: torch.vmap(lin)(a).sum())(x)
+    assert leaf.grad is None
