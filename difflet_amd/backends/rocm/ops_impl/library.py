@@ -142,12 +142,30 @@ def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, sca
 GEMV_ROWS = 8
 
 
-def _gemv_fits(m: int, k: int, n: int) -> bool:
-    """The GEMV kernel stages m rows of x in LDS: m (rounded up to 1, 2, 4 or 8) x k <= 16384. From
-    two rows on its reads of x bound it (3072 x 18432: 2 rows 34 us, 4 rows 56, the GEMM's 64-row
-    tiles 26), so there it keeps the widths the GEMM would have to pad the weight for."""
-    return (m <= GEMV_ROWS and k % 8 == 0 and (m == 1 or k % 64 != 0 or n % 4 != 0)
+def _gemv_stages(m: int, k: int) -> bool:
+    """The GEMV kernel stages m rows of x in LDS: m (rounded up to 1, 2, 4 or 8) x k <= 16384."""
+    return (m <= GEMV_ROWS and k % 8 == 0
             and {1: 1, 2: 2}.get(m, 4 if m <= 4 else 8) * k <= 16384)
+
+
+def _gemv_fits(m: int, k: int, n: int) -> bool:
+    """Whether the GEMV is the faster kernel. From two rows on its reads of x bound it (3072 x 18432:
+    2 rows 34 us, 4 rows 56, the GEMM's 64-row tiles 26), so there it keeps the widths the GEMM
+    would have to pad the weight for."""
+    return _gemv_stages(m, k) and (m == 1 or k % 64 != 0 or n % 4 != 0)
+
+
+def _gemm_reads(x: Tensor, w: Tensor, bias: Optional[Tensor]) -> bool:
+    """Whether the GEMM takes these operands: rows of x that do not overlap and start at multiples of
+    16 bytes (x with strided columns is copied first), a bias at a multiple of 8, operands below
+    4 GiB. The GEMV copies x, reads the bias value by value and takes a weight of any size."""
+    if x.dtype is not torch.bfloat16 or w.shape[0] * w.stride(0) >= 1 << 31:
+        return False
+    if x.stride(1) == 1 and not (x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
+                                 and x.shape[0] * x.stride(0) < 1 << 31 and x.data_ptr() % 16 == 0):
+        return False
+    return bias is None or (bias.dtype is torch.bfloat16 and bias.stride(0) == 1
+                            and bias.data_ptr() % 8 == 0)
 
 
 def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
@@ -157,7 +175,8 @@ def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int
     n_pad, k_pad = w.shape
     if m == 0:
         return x.new_empty((0, out_features), dtype=torch.bfloat16)
-    if n_pad == out_features and k_pad == kx and _gemv_fits(m, kx, n_pad):
+    if n_pad == out_features and k_pad == kx and (
+            _gemv_fits(m, kx, n_pad) or (_gemv_stages(m, kx) and not _gemm_reads(x, w, bias))):
         return kernels.gemv(x, w, bias)
     if kx != k_pad:
         x = F.pad(x, (0, k_pad - kx))

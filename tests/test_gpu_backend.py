@@ -106,6 +106,41 @@ def test_ops_linear_modules(gpu, m, k, n):
     assert rel_l2(y, F.linear(x.float(), row.weight.float().cpu())) < 4e-3
 
 
+@pytest.mark.parametrize("m", [2, 4, 8])
+def test_ops_linear_of_few_rows_takes_any_layout(gpu, m):
+    """2 to 8 rows laid out as no GEMM operand may be: one row expanded, row strides and bases off 16
+    bytes, strided columns, a bias off 8 bytes."""
+    from difflet_amd.backends.rocm.ops_impl import linear as L
+
+    k, n = 2048, 384
+    g = torch.Generator().manual_seed(m)
+    buf = torch.randn(m, 2 * k + 2, generator=g).bfloat16().to(gpu)
+    col = L.ColumnParallelLinear(k, n, dtype=torch.bfloat16).to(gpu)
+    b = torch.randn(n + 1, generator=g).bfloat16().to(gpu)
+    layouts = {"rows": buf[:, :k].contiguous(), "expanded": buf[:1, :k].contiguous().expand(m, k),
+               "row stride": buf[:, :k], "base": buf[:, 1:k + 1],
+               "base of whole rows": torch.cat([buf.flatten()])[1:m * k + 1].view(m, k),
+               "columns": buf[:, 1:2 * k + 1:2], "transposed": buf[:, :k].t().contiguous().t()}
+    for name, x in layouts.items():
+        for bias in (b[:n], b[1:]):
+            print(f"few rows m={m} {name} bias offset {bias.storage_offset()}", flush=True)
+            col.bias = torch.nn.Parameter(bias, requires_grad=False)
+            ref = F.linear(x.float(), col.weight.detach().float(), bias.float())
+            assert rel_l2(col(x), ref) < 4e-3
+
+
+def test_ops_linear_of_few_rows_takes_a_weight_above_4_gib(gpu):
+    from difflet_amd.backends.rocm.ops_impl import library
+
+    k, n = 8192, (1 << 18) + 8
+    g = torch.Generator(device=gpu).manual_seed(1)
+    w = torch.empty(n, k, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    x = torch.empty(2, k, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    y = library.linear(x, w, None, n)
+    for cols in (slice(0, 64), slice(n - 64, n)):  # the last 8 rows lie past 4 GiB
+        assert rel_l2(y[:, cols], F.linear(x.float(), w[cols].float())) < 4e-3
+
+
 @pytest.mark.parametrize("m,k,n", [(3, 3072, 500), (300, 256, 128), (77, 100, 30), (512, 4096, 10240)])
 def test_ops_linear_modules_fp32_weights(gpu, m, k, n):
     """fp32 weights run the fp32 GEMM (K / N off multiples of 4 padded on the weight), fp32
