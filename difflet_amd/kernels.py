@@ -797,8 +797,8 @@ def gemv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
     n = w.shape[0]
     if w.dtype != torch.bfloat16 or w.stride(1) != 1:
         raise TypeError("gemv weights must be bf16 with contiguous rows")
-    if bias is not None and bias.dtype != x2.dtype:
-        bias = bias.to(x2.dtype)
+    if bias is not None:  # the kernel reads n values in a row
+        bias = bias.to(x2.dtype).contiguous()
     y = out if out is not None else torch.empty((m, n), dtype=x2.dtype, device=dev)
     check(lib().difflet_rocm_gemv(_ptr(x2), _dt(x2), m, k, x2.stride(0), _ptr(w), w.stride(0), n,
                                   _ptr(bias), _ptr(y), y.stride(0), int(act), _stream(dev)),

@@ -106,24 +106,24 @@ def test_ops_linear_modules(gpu, m, k, n):
     assert rel_l2(y, F.linear(x.float(), row.weight.float().cpu())) < 4e-3
 
 
-@pytest.mark.parametrize("m", [2, 4, 8])
+@pytest.mark.parametrize("m", [1, 2, 4, 8])
 def test_ops_linear_of_few_rows_takes_any_layout(gpu, m):
-    """2 to 8 rows laid out as no GEMM operand may be: one row expanded, row strides and bases off 16
-    bytes, strided columns, a bias off 8 bytes."""
+    """Few rows laid out as no GEMM operand may be: one row expanded, row strides and bases off 16
+    bytes, strided columns, a bias off 8 bytes or strided."""
     from difflet_amd.backends.rocm.ops_impl import linear as L
 
     k, n = 2048, 384
     g = torch.Generator().manual_seed(m)
     buf = torch.randn(m, 2 * k + 2, generator=g).bfloat16().to(gpu)
     col = L.ColumnParallelLinear(k, n, dtype=torch.bfloat16).to(gpu)
-    b = torch.randn(n + 1, generator=g).bfloat16().to(gpu)
+    b = torch.randn(2 * n, generator=g).bfloat16().to(gpu)
     layouts = {"rows": buf[:, :k].contiguous(), "expanded": buf[:1, :k].contiguous().expand(m, k),
                "row stride": buf[:, :k], "base": buf[:, 1:k + 1],
                "base of whole rows": torch.cat([buf.flatten()])[1:m * k + 1].view(m, k),
                "columns": buf[:, 1:2 * k + 1:2], "transposed": buf[:, :k].t().contiguous().t()}
     for name, x in layouts.items():
-        for bias in (b[:n], b[1:]):
-            print(f"few rows m={m} {name} bias offset {bias.storage_offset()}", flush=True)
+        for bias in (b[:n], b[1:n + 1], b[::2]):
+            print(f"few rows m={m} {name} bias {bias.storage_offset()} {bias.stride(0)}", flush=True)
             col.bias = torch.nn.Parameter(bias, requires_grad=False)
             ref = F.linear(x.float(), col.weight.detach().float(), bias.float())
             assert rel_l2(col(x), ref) < 4e-3
