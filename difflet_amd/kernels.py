@@ -365,13 +365,26 @@ def _check_qk(qk: QkNormRope, problems: Sequence[Problem]) -> None:
             raise ValueError(f"problem {i}: RoPE rows [{lo}, {hi}) exceed the {rows}-row tables")
 
 
+def _launch_scratch(kind: str, m: int, n: int, k: int, dev: torch.device) -> torch.Tensor | None:
+    """Scratch of one launch (difflet_rocm_gemm_scratch_bytes: up to 64 MB for K pieces, 134 MB on
+    256 compute units for a cut last wave), from torch's allocator and returned to it with the
+    call. None where no scratch helps or the memory is not there: the launch then keeps K whole."""
+    nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID[kind], m, n, k)
+    if not nbytes:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
                  epilogue: int = _lib.EPI_NONE, act_col_start: int = 0,
                  workspace: torch.Tensor | None | str = None,
                  qk: QkNormRope | None = None) -> None:
     """Runs up to 4 GEMMs sharing N, K and the epilogue in one launch (writes each p.c).
     workspace: None (every tile whole on one workgroup, the default), "call" (scratch of this
-    call alone, from torch's allocator, where a launch of few tiles gains by cutting K: safe on
+    call alone, from torch's allocator, where the launch gains by it, see _launch_scratch: safe on
     any stream and under graph capture), "shared" (the current stream's, see gemm_workspace) or
     a zero-filled uint8 tensor of
     difflet_rocm_gemm_workspace_bytes() bytes, which lets a launch whose last wave of tiles
@@ -447,10 +460,9 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
             workspace = None
             if len(problems) == 1 and qk is None and epilogue in (_lib.EPI_NONE,
                                                                   _lib.EPI_GATE_RESIDUAL):
-                nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID[kind], arr[0].m, n, k)
+                workspace = _launch_scratch(kind, arr[0].m, n, k, dev)
                 # a buffer large enough for the split schedule needs its counters zeroed here
-                if nbytes:
-                    workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+                if workspace is not None:
                     workspace[:_COUNTER_BYTES].zero_()
         else:
             raise ValueError("workspace must be 'shared', 'call', a tensor or None, "
@@ -506,14 +518,12 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
         gemm_grouped([Problem(a, w, y, bias, a_scale=a_scale, w_scale=w_scale)], kind=kind,
                      workspace="call")
         return y
-    c = lib()
-    nbytes = c.difflet_rocm_gemm_scratch_bytes(kid, m, n, k)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
-    check(c.difflet_rocm_gemm_single(
+    ws = _launch_scratch(kind, m, n, k, dev)
+    check(lib().difflet_rocm_gemm_single(
         kid, a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), n,
         None if bias is None else bias.data_ptr(), a_scale.data_ptr() if kid else None,
-        w_scale.data_ptr() if kid else None, m, n, k, None if ws is None else ws.data_ptr(), nbytes,
-        _raw_stream(dev)), f"gemm_{kind}")
+        w_scale.data_ptr() if kid else None, m, n, k, None if ws is None else ws.data_ptr(),
+        0 if ws is None else ws.numel(), _raw_stream(dev)), f"gemm_{kind}")
     return y
 
 
@@ -864,8 +874,7 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
     y = out if out is not None else torch.empty((m, n), dtype=torch.float32, device=dev)
     scratch = None
     if workspace == "call":
-        nbytes = lib().difflet_rocm_gemm_scratch_bytes(_KIND_ID["f32"], m, n, k)
-        scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        scratch = _launch_scratch("f32", m, n, k, dev)
     elif workspace is not None:
         raise ValueError(f"workspace must be 'call' or None, got {workspace!r}")
     check(lib().difflet_rocm_gemm_f32_scratch(

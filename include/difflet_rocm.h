@@ -237,7 +237,8 @@ int64_t difflet_rocm_gemm_workspace_bytes(void);
 /* Bytes of scratch with which one m x n x k problem (kind 0 bf16, 1 fp8 per row, 2 MXFP8, 3
  * fp32; epilogue NONE or GATE_RESIDUAL) runs at its fastest among the small-launch plans: passed as the
  * workspace of difflet_rocm_gemm_single or difflet_rocm_gemm_f32_scratch, not zeroed, used by that
- * launch only. 0: no scratch helps. */
+ * launch only. At most 64 MiB for K pieces, difflet_rocm_gemm_workspace_bytes() for a cut last
+ * wave. 0: no scratch helps. */
 int64_t difflet_rocm_gemm_scratch_bytes(int kind, int64_t m, int64_t n, int64_t k);
 
 /* One problem with EPI_NONE through the GEMM of `kind` (0 bf16, 1 fp8 per row, 2 MXFP8), its

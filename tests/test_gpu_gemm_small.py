@@ -118,3 +118,42 @@ def test_linear_call_split_schedule_on_scratch(gpu, kind, m, n, k):
     kernels.gemm_grouped([kernels.Problem(aq, wq, whole, a_scale=sa, w_scale=sw)], kind=kind)
     d = (outs[0].float() - whole.float()).norm() / whole.float().norm()
     assert d.item() < 2e-3
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 128, 3072, 12288), ("bf16", 6889, 3072, 6144),
+                                        ("fp8", 6889, 3072, 12288), ("f32", 16, 4096, 4096)])
+def test_calls_without_memory_for_scratch(gpu, monkeypatch, kind, m, n, k):
+    """Scratch only saves time: where torch has no memory for it the call runs with K whole, equal up
+    to the order of fp32 sums (a bf16 step, 2e-3; fp32 1e-5)."""
+    print(f"no scratch {kind} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(m)
+    a, w = rnd(g, m, k), rnd(g, n, k, std=0.05)
+    kid = {"bf16": 0, "fp8": 1, "mx": 2, "f32": 3}[kind]
+    assert _lib.load().difflet_rocm_gemm_scratch_bytes(kid, m, n, k) > 0
+    if kind == "f32":
+        a, w = a.float().to(gpu), w.float().to(gpu)
+        calls = [lambda: kernels.gemm_f32(a, w, workspace="call")]
+    else:
+        aq, wq, sa, sw = _operands(kind, a, w, gpu)
+
+        def grouped():
+            c = torch.empty(m, n, dtype=torch.bfloat16, device=gpu)
+            kernels.gemm_grouped([kernels.Problem(aq, wq, c, a_scale=sa, w_scale=sw)], kind=kind,
+                                 workspace="call")
+            return c
+
+        calls = [grouped, lambda: kernels.gemm_call(kind, aq, wq, None, sa, sw)]
+    want = [f() for f in calls]
+    empty = torch.empty
+
+    def no_scratch(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no memory left")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", no_scratch)
+    got = [f() for f in calls]
+    monkeypatch.undo()
+    for x, y in zip(got, want):
+        d = (x.float() - y.float()).norm() / y.float().norm()
+        assert d.item() < (1e-5 if kind == "f32" else 2e-3)
