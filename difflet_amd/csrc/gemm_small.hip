@@ -186,20 +186,25 @@ __global__ __launch_bounds__(BN == 64 ? 256 : 512, 1) void gemm_small_kernel(
   const int nkt = min(args.piece_stages, nk - kbeg);
 
   const int64_t arow = args.lda * EB, wrow = args.ldw * EB;
-  const i32x4 ra = rsrc_of(args.a + m0 * arow, (int64_t)(M - m0) * arow);
-  const i32x4 rw = rsrc_of(args.w + n0 * wrow, (int64_t)(N - n0) * wrow);
-  // lane l of a 1 KB load fills slab row l / 8, chunk l % 8; rows past M or N read zero
+  // the buffers end with the tile's last row, not a row stride after it (rows may be a column
+  // range of wider ones), and never reach kOut: gemm.hip admits operands of up to 2^32 - 16 bytes,
+  // fp32 rows are below 2^24
+  constexpr uint32_t kOut = 0xfffffff0u;
+  const int arows = min(M - m0, BM), wrows = min(N - n0, BN);
+  const i32x4 ra = rsrc_of(args.a + m0 * arow, (arows - 1) * arow + (int64_t)args.k * EB);
+  const i32x4 rw = rsrc_of(args.w + n0 * wrow, (wrows - 1) * wrow + (int64_t)args.k * EB);
+  // lane l of a 1 KB load fills slab row l / 8, chunk l % 8; rows past M or N read zero, at kOut:
+  // where rows are 16 MB and more apart (one token of each batch element) their own offsets would
+  // wrap to ones that another row covers
   uint32_t aoff[4], woff[4];
+  auto row_off = [&](int r, int rows, int64_t row) {
+    const uint32_t o = (uint32_t)r * (uint32_t)row + (uint32_t)(((lane & 7) ^ swz8s(r)) << 4);
+    return r < rows ? o : kOut;
+  };
 #pragma unroll
-  for (int i = 0; i < SA; ++i) {
-    const int r = (wave * SA + i) * 8 + (lane >> 3);
-    aoff[i] = (uint32_t)(r * arow) + (uint32_t)(((lane & 7) ^ swz8s(r)) << 4);
-  }
+  for (int i = 0; i < SA; ++i) aoff[i] = row_off((wave * SA + i) * 8 + (lane >> 3), arows, arow);
 #pragma unroll
-  for (int i = 0; i < SW; ++i) {
-    const int r = (wave * SW + i) * 8 + (lane >> 3);
-    woff[i] = (uint32_t)(r * wrow) + (uint32_t)(((lane & 7) ^ swz8s(r)) << 4);
-  }
+  for (int i = 0; i < SW; ++i) woff[i] = row_off((wave * SW + i) * 8 + (lane >> 3), wrows, wrow);
   const int ksb = args.k / 32;  // MX: scale bytes per row
   i32x4 rsa = ra, rsw = rw;
   if constexpr (E == SmallElem::MX) {
@@ -220,7 +225,8 @@ __global__ __launch_bounds__(BN == 64 ? 256 : 512, 1) void gemm_small_kernel(
     }
   };
   // stage kt's loads into slot st; past the piece's last stage they are issued with an offset
-  // beyond both buffers (zeros, no memory traffic), so every barrier waits with one vmcnt
+  // beyond all but the largest buffers (zeros, no memory traffic), so every barrier waits with one
+  // vmcnt; what a larger one returns there is not used
   auto issue = [&](int kt, int st) {
     const uint32_t kb = kt < nkt ? (uint32_t)(kbeg + kt) * 128u : 0u;
     const uint32_t off = kt < nkt ? 0u : 0x80000000u;
@@ -230,7 +236,7 @@ __global__ __launch_bounds__(BN == 64 ? 256 : 512, 1) void gemm_small_kernel(
       if constexpr (F32) {
         const int r = slab * 8 + (lane >> 3);
         const int kk = (kbeg + kt) * 32 + ((lane & 7) ^ swz8s(r)) * 4;
-        return kt < nkt && kk < args.k ? o : 0xfffffff0u;
+        return kt < nkt && kk < args.k ? o : kOut;
       }
       return o | off;
     };

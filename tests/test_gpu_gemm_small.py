@@ -157,3 +157,33 @@ def test_calls_without_memory_for_scratch(gpu, monkeypatch, kind, m, n, k):
     for x, y in zip(got, want):
         d = (x.float() - y.float()).norm() / y.float().norm()
         assert d.item() < (1e-5 if kind == "f32" else 2e-3)
+
+
+@pytest.mark.parametrize("m,s,k", [(2, 32760, 5120), (5, 16384, 3072), (70, 8400, 2048)])
+def test_rows_far_apart(gpu, m, s, k):
+    """The last token of each of m batch elements: rows 34 to 335 MB apart, so that a tile's rows past
+    m would lie 4 GiB and more past its first. The GEMM's tiles and the linear op's."""
+    from difflet_amd.backends.rocm.ops_impl import library
+
+    print(f"rows far apart m={m} s={s} k={k}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m)
+    x = torch.empty(m, s, k, dtype=torch.bfloat16, device=gpu)[:, -1]
+    x.normal_(generator=g)
+    w = torch.empty(384, k, dtype=torch.bfloat16, device=gpu).normal_(std=0.05, generator=g)
+    want = kernels.gemm_call("bf16", x.contiguous(), w, None)
+    assert rel_l2(want, x.float() @ w.float().t()) < TOL
+    assert torch.equal(kernels.gemm_call("bf16", x, w, None), want)
+    assert torch.equal(library.linear(x, w, None, 384), want)
+
+
+def test_fp32_gemm_above_4_gib(gpu):
+    """A weight past 4 GiB and K off the 32-float stage: the stage's missing values are zeros, not the
+    weight's 2^32 - 16 bytes on (infinite here in row 1044495, which every row but its own ignores)."""
+    n, k, hit = (1 << 20) + 64, 1028, (1 << 32) // (1028 * 4)
+    w = torch.full((n, k), 0.5, device=gpu)
+    w[hit] = float("inf")
+    a = torch.ones(3, k, device=gpu)
+    y = kernels.gemm_f32(a, w, workspace="call")
+    assert torch.isinf(y[:, hit]).all()
+    y[:, hit] = 0.5 * k
+    assert bool((y == 0.5 * k).all())  # sums of halves: exact
