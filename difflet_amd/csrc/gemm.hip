@@ -1254,6 +1254,11 @@ static int gemm_launch(const char* name, int nproblems, const difflet_gemm_probl
       return dlt_check_launch(name);
     }
   }
+  // the kernel addresses the 256 rows of a tile, also those past m or n, in 32 bits: farther apart
+  // (fewer than 256 of them then, by the 4 GiB bound) they would wrap onto other memory
+  for (int i = 0; i < nproblems; ++i)
+    DLT_REQUIRE(BM * problems[i].lda * EB <= (1LL << 32) && BN * problems[i].ldw * EB <= (1LL << 32),
+                DIFFLET_EUNSUPPORTED, "%s: rows of problem %d lie more than 16 MB apart", name, i);
   args.ws = (uint8_t*)workspace;
   constexpr int NT = ElemTraits<E>::WN;
   dim3 grid((unsigned)(args.sk.dp + args.sk.groups)), block(128 * NT);

@@ -365,6 +365,14 @@ def _check_qk(qk: QkNormRope, problems: Sequence[Problem]) -> None:
             raise ValueError(f"problem {i}: RoPE rows [{lo}, {hi}) exceed the {rows}-row tables")
 
 
+def _near_rows(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy of it where its rows are over 16 MB apart (fewer than 256 rows, below the GEMMs'
+    4 GiB: one token of each batch element, say), which the GEMM kernels do not address."""
+    if t.dim() == 2 and t.stride(0) * t.element_size() > 1 << 24 and t.shape[0] < 256:
+        return t.contiguous()
+    return t
+
+
 def _launch_scratch(kind: str, m: int, n: int, k: int, dev: torch.device) -> torch.Tensor | None:
     """Scratch of one launch (difflet_rocm_gemm_scratch_bytes: up to 64 MB for K pieces, 134 MB on
     256 compute units for a cut last wave), from torch's allocator and returned to it with the
@@ -432,10 +440,12 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
         _check_qk(qk, problems)
     dev = _on_gpu(*[t for p in problems for t in (p.a, p.w, p.c, p.bias, p.gate, p.residual,
                                                   p.a_scale, p.w_scale)])
+    operands = [(_near_rows(p.a), _near_rows(p.w)) for p in problems]
     for i, p in enumerate(problems):
         q = arr[i]
-        q.a, q.lda = p.a.data_ptr(), p.a.stride(0)
-        q.w, q.ldw = p.w.data_ptr(), p.w.stride(0)
+        a, w = operands[i]
+        q.a, q.lda = a.data_ptr(), a.stride(0)
+        q.w, q.ldw = w.data_ptr(), w.stride(0)
         q.c, q.ldc = p.c.data_ptr(), p.c.stride(0)
         q.bias = p.bias.data_ptr() if p.bias is not None else None
         if p.gate is not None:
@@ -495,6 +505,7 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
     m, k = a.shape[0], w.shape[-1]
     n = w.shape[0]
     dev = a.device
+    a, w = _near_rows(a), _near_rows(w)
     y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
     kid = _KIND_ID[kind]
 

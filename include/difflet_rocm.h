@@ -173,7 +173,8 @@ enum difflet_epilogue {
 };
 
 typedef struct difflet_gemm_problem {
-  const void* a;        /* [m, k], row stride lda (bf16, or e4m3 codes for the fp8 GEMMs) */
+  const void* a;        /* [m, k], row stride lda (bf16, or e4m3 codes for the fp8 GEMMs); rows of a
+                         * and w lie at most 16 MB apart */
   int64_t lda;
   const void* w;        /* [n, k], row stride ldw */
   int64_t ldw;

@@ -153,3 +153,27 @@ def test_fp32_output_epilogue_checks():
              _lib.EPI_F32)
     with pytest.raises(ValueError, match="bf16 GEMM"):
         _run(_prob("fp8"), "fp8", _lib.EPI_F32)
+
+
+@pytest.mark.parametrize("kind,eb", [("bf16", 2), ("fp8_rowwise", 1), ("mxfp8", 1)])
+@pytest.mark.parametrize("operand", ["lda", "ldw"])
+def test_the_c_abi_refuses_rows_its_tiles_cannot_address(kind, eb, operand):
+    """Rows past m or n of a 256-row tile are addressed too, in 32 bits: over 16 MB apart, their
+    offsets would wrap onto other memory (placeholder addresses: the call fails in validation)."""
+    fn = getattr(_lib.load(), f"difflet_rocm_gemm_{kind}")
+    fake = 1 << 20
+    probs = (_lib.GemmProblem * 1)()
+    p = probs[0]
+    p.a, p.w, p.c, p.a_scale, p.w_scale = fake, fake, fake, fake, fake
+    p.lda, p.ldw, p.ldc, p.m, p.rows_per_batch = K, K, 128, 12, 12
+    setattr(p, operand, ((1 << 24) + 128) // eb)
+    st = fn(1, probs, 128, K, _lib.EPI_GELU, 0, None, 0, None, None)
+    assert st == _lib.EUNSUPPORTED
+    assert b"more than 16 MB apart" in _lib.load().difflet_rocm_last_error()
+
+
+def test_rows_far_apart_are_copied():
+    far = torch.empty_strided((3, K), ((1 << 23) + 64, 1), dtype=torch.bfloat16, device="meta")
+    near = torch.empty_strided((3, K), (1 << 23, 1), dtype=torch.bfloat16, device="meta")
+    assert kernels._near_rows(far).stride() == (K, 1)
+    assert kernels._near_rows(near) is near

@@ -162,7 +162,8 @@ def test_calls_without_memory_for_scratch(gpu, monkeypatch, kind, m, n, k):
 @pytest.mark.parametrize("m,s,k", [(2, 32760, 5120), (5, 16384, 3072), (70, 8400, 2048)])
 def test_rows_far_apart(gpu, m, s, k):
     """The last token of each of m batch elements: rows 34 to 335 MB apart, so that a tile's rows past
-    m would lie 4 GiB and more past its first. The GEMM's tiles and the linear op's."""
+    m would lie 4 GiB and more past its first. Small tiles, the linear op's, and with two problems
+    in a launch the 256 x 256 ones."""
     from difflet_amd.backends.rocm.ops_impl import library
 
     print(f"rows far apart m={m} s={s} k={k}", flush=True)
@@ -174,6 +175,12 @@ def test_rows_far_apart(gpu, m, s, k):
     assert rel_l2(want, x.float() @ w.float().t()) < TOL
     assert torch.equal(kernels.gemm_call("bf16", x, w, None), want)
     assert torch.equal(library.linear(x, w, None, 384), want)
+    c = [torch.empty_like(want) for _ in range(4)]
+    kernels.gemm_grouped([kernels.Problem(t, w, y) for t, y in zip((x, x.contiguous()), c[:2])])
+    kernels.linear(x, w, epilogue=_lib.EPI_GELU, out=c[2])
+    kernels.linear(x.contiguous(), w, epilogue=_lib.EPI_GELU, out=c[3])
+    assert torch.equal(c[0], c[1]) and torch.equal(c[2], c[3])
+    assert rel_l2(c[0], want.float()) < TOL
 
 
 def test_fp32_gemm_above_4_gib(gpu):
