@@ -6,13 +6,14 @@
 //
 // Activations are channels-last: [batch][pixels][channels], pixels row-major (y * W + x).
 //
-// GroupNorm runs in two passes over the activation: per-chunk, per-channel means and sums of
-// squared deviations, merged per (batch, group) in double precision, then the normalization
-// with the affine weights (and SiLU) applied elementwise. The deviations are taken from running
-// means (Welford's update, four pixels at a time), which keeps the variance free of the
-// E[x^2] - E[x]^2 cancellation in one read; both statistics are the population ones of
-// F.group_norm. Both passes are bound by HBM. With the variance in a read of its own the FLUX
-// decoder's 30 norms took 4.55 ms of a 1024 x 1024 decode, 2.9 now.
+// GroupNorm runs in two passes over the activation: per-chunk sums of each group's values and of
+// their squares, relative to the group's first value and in double precision, then the
+// normalization with the affine weights (and SiLU) applied elementwise. Products of shifted values
+// are exact or rounded at 2^-53, so one read gives the variance free of the E[x^2] - E[x]^2
+// cancellation; both statistics are the population ones of F.group_norm. Both passes are bound by
+// HBM, the sums too: double precision adds as fast as single on this part, and took less than the
+// running means and deviations in fp32 before it (128 channels of 1024 x 1024 pixels with SiLU in
+// bf16 203 -> 181 us, 4.4 TB/s; fp32 340 -> 338 us).
 
 #include <hip/hip_runtime.h>
 
@@ -57,140 +58,112 @@ template <> struct Vec8<float> {
   }
 };
 
-// Mean and sum of squared deviations of a part of n values merged into those of m others.
-__device__ __forceinline__ void gn_merge(float& mean, float& m2, float m, float pmean, float pm2,
-                                         float n) {
-  const float d = pmean - mean, f = n / (m + n);
-  mean = __builtin_fmaf(d, f, mean);
-  m2 += __builtin_fmaf(d * d, m * f, pm2);
+// The value that a group's sums are relative to: its first of the batch element.
+template <typename T>
+__device__ __forceinline__ double gn_shift(const T* x, int64_t pixels, int channels, int b, int c0) {
+  return (double)Elt<T>::load(x + (int64_t)b * pixels * channels + c0);
 }
 
-// ---- GroupNorm pass 1: per channel, the mean and the sum of squared deviations over a chunk of
+// ---- GroupNorm pass 1: per group, the sums of x - shift and of (x - shift)^2 over a chunk of
 // pixels. Thread t handles channels 8 (t % tpp) .. + 8 of pixel t / tpp of each pass (tpp = C / 8
-// threads per pixel), four pixels' loads in flight; the workgroup's threads that share channels
-// merge through LDS, then each group's channels. partial: [batch][chunks][2][groups] (means, sums).
+// threads per pixel), four pixels' loads in flight; the threads that share channels are summed
+// through LDS, then each group's channels. partial: [batch][chunks][2][groups].
 template <typename T>
 __global__ __launch_bounds__(256) void gn_stats_kernel(const T* __restrict__ x, int64_t pixels,
                                                        int channels, int groups, int64_t chunk,
-                                                       float* __restrict__ partial) {
-  __shared__ float red[256][17];
+                                                       double* __restrict__ partial) {
+  __shared__ double red[16][256];  // [sum 0 .. 7, sum of squares 0 .. 7][thread]
   const int tid = threadIdx.x, tpp = channels / 8, ppass = 256 / tpp;
   const int b = blockIdx.y, ck = blockIdx.x;
   const int cv = tid % tpp, pr = tid / tpp;
-  const bool active = pr < ppass;
-  float mean[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  float m2[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const int cpg = channels / groups;
+  double shift[8], s1[8], s2[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    shift[i] = gn_shift(x, pixels, channels, b, (cv * 8 + i) / cpg * cpg);
+    s1[i] = s2[i] = 0.0;
+  }
   const int64_t p0 = ck * chunk, p1 = min(p0 + chunk, pixels);
   const T* xb = x + (int64_t)b * pixels * channels + cv * 8;
-  if (active) {
-    float n = 0.f;
+  auto add = [&](const float* v) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double d = (double)v[i] - shift[i];
+      s1[i] += d;
+      s2[i] = __builtin_fma(d, d, s2[i]);
+    }
+  };
+  if (pr < ppass) {
     int64_t p = p0 + pr;
     for (; p + 3 * ppass < p1; p += 4 * ppass) {
       float v[4][8];
 #pragma unroll
       for (int u = 0; u < 4; ++u) Vec8<T>::load(xb + (p + u * ppass) * channels, v[u]);
-      const float f = 4.f * __builtin_amdgcn_rcpf(n + 4.f), nf = n * f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q = 0.25f * ((v[0][i] + v[1][i]) + (v[2][i] + v[3][i]));
-        float e = 0.f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) e = __builtin_fmaf(v[u][i] - q, v[u][i] - q, e);
-        const float d = q - mean[i];
-        mean[i] = __builtin_fmaf(d, f, mean[i]);
-        m2[i] += __builtin_fmaf(d * d, nf, e);
-      }
-      n += 4.f;
+      for (int u = 0; u < 4; ++u) add(v[u]);
     }
     for (; p < p1; p += ppass) {
       float v[8];
       Vec8<T>::load(xb + p * channels, v);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) gn_merge(mean[i], m2[i], n, v[i], 0.f, 1.f);
-      n += 1.f;
+      add(v);
     }
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    red[tid][i] = mean[i];
-    red[tid][8 + i] = m2[i];
+    red[i][tid] = s1[i];
+    red[8 + i][tid] = s2[i];
   }
   __syncthreads();
-  if (tid < tpp) {  // threads tid, tid + tpp, ..: row r has the pixels p0 + r, p0 + r + ppass, ..
-    float n = 0.f;
-    for (int r = 0; r < ppass; ++r) {
-      const int64_t left = p1 - p0 - r;
-      if (left <= 0) break;
-      const float nr = (float)((left + ppass - 1) / ppass);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (r == 0) {
-          mean[i] = red[tid][i];
-          m2[i] = red[tid][8 + i];
-        } else {
-          gn_merge(mean[i], m2[i], n, red[r * tpp + tid][i], red[r * tpp + tid][8 + i], nr);
-        }
-      }
-      n += nr;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {  // row 0 of a thread's channels is its own: no one else reads it
-      red[tid][i] = mean[i];
-      red[tid][8 + i] = m2[i];
-    }
+  for (int e = tid; e < 2 * channels; e += 256) {  // one sum of a channel: threads c / 8 + r tpp
+    const int c = e % channels, row = (c & 7) + 8 * (e / channels);
+    double s = red[row][c >> 3];
+    for (int r = 1; r < ppass; ++r) s += red[row][r * tpp + (c >> 3)];
+    red[row][c >> 3] = s;
   }
   __syncthreads();
-  const int cpg = channels / groups;
-  const float n = (float)(p1 - p0);  // per channel
-  float* out = partial + ((int64_t)b * gridDim.x + ck) * 2 * groups;
-  for (int g = tid; g < groups; g += 256) {
-    const int c0 = g * cpg;
-    float gm = red[c0 >> 3][c0 & 7], g2 = red[c0 >> 3][8 + (c0 & 7)];
-    for (int k = 1; k < cpg; ++k)
-      gn_merge(gm, g2, (float)k * n, red[(c0 + k) >> 3][(c0 + k) & 7],
-               red[(c0 + k) >> 3][8 + ((c0 + k) & 7)], n);
-    out[g] = gm;
-    out[groups + g] = g2;
+  double* out = partial + ((int64_t)b * gridDim.x + ck) * 2 * groups;
+  for (int e = tid; e < 2 * groups; e += 256) {
+    const int c0 = e % groups * cpg, half = 8 * (e / groups);
+    double s = 0.0;
+    for (int c = c0; c < c0 + cpg; ++c) s += red[half + (c & 7)][c >> 3];
+    out[e] = s;
   }
 }
 
-// One workgroup per (batch, group): the chunks' means and sums merged in double: the mean of all, then the sum of the parts' deviations and of their means' from it.
-// mean_out, rstd_out = 1 / sqrt(var + eps).
-__global__ __launch_bounds__(256) void gn_reduce_kernel(const float* __restrict__ partial,
-                                                        int chunks, int64_t chunk, int channels,
-                                                        int groups, int64_t pixels, float eps,
-                                                        float* __restrict__ mean_out,
+// One workgroup per (batch, group): the chunks' sums added up. mean_out, rstd_out = 1 / sqrt(var +
+// eps).
+template <typename T>
+__global__ __launch_bounds__(256) void gn_reduce_kernel(const double* __restrict__ partial,
+                                                        const T* __restrict__ x, int chunks,
+                                                        int channels, int groups, int64_t pixels,
+                                                        float eps, float* __restrict__ mean_out,
                                                         float* __restrict__ rstd_out) {
-  __shared__ double red[4];
+  __shared__ double red[2][4];
   const int i = blockIdx.x;  // b * groups + g
   const int b = i / groups, gi = i % groups, cpg = channels / groups;
-  const float* base = partial + (int64_t)b * chunks * 2 * groups + gi;
-  auto count = [&](int c) {  // values of chunk c
-    return (double)((c + 1 < chunks ? chunk : pixels - (int64_t)(chunks - 1) * chunk) * cpg);
-  };
-  auto block_sum_d = [&](double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    __syncthreads();  // the previous sum has been read
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return (red[0] + red[1]) + (red[2] + red[3]);
-  };
-  double s = 0.0;
-  for (int c = threadIdx.x; c < chunks; c += 256)
-    s += count(c) * (double)base[(int64_t)c * 2 * groups];
-  const double n = (double)pixels * (double)cpg;
-  const double mean = block_sum_d(s) / n;
-  s = 0.0;
+  const double* base = partial + (int64_t)b * chunks * 2 * groups + gi;
+  double s1 = 0.0, s2 = 0.0;
   for (int c = threadIdx.x; c < chunks; c += 256) {
-    const float* q = base + (int64_t)c * 2 * groups;
-    const double d = (double)q[0] - mean;
-    s += (double)q[groups] + count(c) * d * d;
+    s1 += base[(int64_t)c * 2 * groups];
+    s2 += base[(int64_t)c * 2 * groups + groups];
   }
-  const double var = block_sum_d(s) / n;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    s1 += __shfl_xor(s1, o, kWave);
+    s2 += __shfl_xor(s2, o, kWave);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s1;
+    red[1][threadIdx.x >> 6] = s2;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    mean_out[i] = (float)mean;
-    rstd_out[i] = (float)(1.0 / __builtin_sqrt(var + (double)eps));
+    const double n = (double)pixels * (double)cpg;
+    const double d = ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3])) / n;
+    const double var = ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3])) / n - d * d;
+    mean_out[i] = (float)(gn_shift(x, pixels, channels, b, gi * cpg) + d);
+    // rounding may leave a variance of zero just below it; NaN stays NaN
+    rstd_out[i] = (float)(1.0 / __builtin_sqrt((var < 0.0 ? 0.0 : var) + (double)eps));
   }
 }
 
@@ -480,7 +453,7 @@ extern "C" int64_t difflet_rocm_group_norm_workspace_bytes(int64_t batch, int64_
                                                            int64_t channels, int64_t groups) {
   if (batch <= 0 || pixels <= 0 || channels <= 0 || groups <= 0) return 0;
   const int64_t chunks = (pixels + gn_chunk(pixels, (int)channels) - 1) / gn_chunk(pixels, (int)channels);
-  return (batch * chunks * 2 * groups + 2 * batch * groups) * 4;
+  return batch * chunks * 2 * groups * 8 + 2 * batch * groups * 4;  // sums, means, 1 / deviations
 }
 
 extern "C" int difflet_rocm_group_norm(const void* x, void* y, int dtype, int64_t batch,
@@ -505,8 +478,8 @@ extern "C" int difflet_rocm_group_norm(const void* x, void* y, int dtype, int64_
               (long long)need);
   const int64_t chunk = gn_chunk(pixels, (int)channels);
   const int chunks = (int)((pixels + chunk - 1) / chunk);
-  float* partial = reinterpret_cast<float*>(workspace);
-  float* mean = partial + batch * chunks * 2 * groups;
+  double* partial = reinterpret_cast<double*>(workspace);
+  float* mean = reinterpret_cast<float*>(partial + batch * chunks * 2 * groups);
   float* rstd = mean + batch * groups;
   hipStream_t s = (hipStream_t)stream;
   const dim3 sgrid((unsigned)chunks, (unsigned)batch);
@@ -518,8 +491,8 @@ extern "C" int difflet_rocm_group_norm(const void* x, void* y, int dtype, int64_
   DLT_DISPATCH_BF16_F32(dtype, T,
     hipLaunchKernelGGL((gn_stats_kernel<T>), sgrid, dim3(256), 0, s, (const T*)x, pixels,
                        (int)channels, (int)groups, chunk, partial);
-    hipLaunchKernelGGL(gn_reduce_kernel, dim3(rblocks), dim3(256), 0, s, partial, chunks, chunk,
-                       (int)channels, (int)groups, pixels, eps, mean, rstd);
+    hipLaunchKernelGGL((gn_reduce_kernel<T>), dim3(rblocks), dim3(256), 0, s, partial, (const T*)x,
+                       chunks, (int)channels, (int)groups, pixels, eps, mean, rstd);
     hipLaunchKernelGGL((gn_apply_kernel<T>), agrid, dim3(256), 0, s, (const T*)x, (T*)y, pixels,
                        (int)channels, (int)groups, mean, rstd, weight, bias, act));
   return dlt_check_launch("group_norm");

@@ -961,7 +961,7 @@ def group_norm(x: torch.Tensor, groups: int, weight: torch.Tensor | None,
                bias: torch.Tensor | None, eps: float, *, silu: bool = False,
                out: torch.Tensor | None = None) -> torch.Tensor:
     """GroupNorm (+ SiLU) of channels-last x [batch, pixels, C] (bf16 or fp32) with fp32 affine
-    vectors; statistics in fp32 / double, two passes."""
+    vectors; statistics in double."""
     if x.dim() != 3 or not x.is_contiguous():
         raise ValueError("group_norm: x must be a contiguous [batch, pixels, channels]")
     b, p, c = x.shape

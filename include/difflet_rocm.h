@@ -484,7 +484,7 @@ int64_t difflet_rocm_group_norm_workspace_bytes(int64_t batch, int64_t pixels, i
                                                 int64_t groups);
 
 /* GroupNorm over channels-last x (bf16 or fp32): per (batch, group) mean and population
- * variance in fp32 / double, y = (x - mean) / sqrt(var + eps) * weight + bias (fp32 vectors,
+ * variance in double, y = (x - mean) / sqrt(var + eps) * weight + bias (fp32 vectors,
  * either may be null), then SiLU when act == 1. PatchedGroupNorm / nn.GroupNorm + SiLU of the
  * decoder's resnets and output (modeling_vae.py:39-68: F.group_norm in fp32). channels a
  * multiple of 8 and of groups, <= 2048; y may alias x. */

@@ -10,7 +10,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from difflet_amd import kernels
+from difflet_amd import _lib, kernels
 from difflet_amd.vae import decoder as dvae
 from oracle import vae as ovae
 
@@ -41,6 +41,33 @@ def test_group_norm_matches_torch(gpu, dtype, c, pix):
     assert out.dtype == dtype and rel_l2(out, ref) < tol
     out = kernels.group_norm(x.to(gpu), groups, w.to(gpu), b.to(gpu), 1e-6, silu=True)
     assert rel_l2(out, F.silu(ref)) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("c,pix", [(128, 70001), (512, 4096), (24, 5000), (2048, 130), (256, 1)])
+@pytest.mark.parametrize("mean", [0.0, 3.0, 1000.0])
+def test_group_norm_statistics_are_those_of_64_bits(gpu, dtype, c, pix, mean):
+    """The mean and 1 / deviation that the normalization multiplies by, at the workspace's end: the
+    64-bit statistics rounded once to fp32 (half a unit in the last place; sums of up to 2^21 values
+    err by 2^21 2^-53 of the values' spread, under 0.01 units of the results). Constant groups too."""
+    print(f"group norm statistics {dtype} {c} {pix} {mean}", flush=True)
+    g = torch.Generator().manual_seed(c + pix)
+    groups, eps = (32 if c % 32 == 0 else 8), 1e-6
+    x = (torch.randn(2, pix, c, generator=g) + mean).to(dtype)
+    x[1, :, : c // groups] = x[1, 0, 0]  # one group without variance
+    xg = x.to(gpu)
+    lib = _lib.load()
+    need = lib.difflet_rocm_group_norm_workspace_bytes(2, pix, c, groups)
+    ws = torch.full((need,), 0xff, dtype=torch.uint8, device=gpu)
+    dt = _lib.F32 if dtype == torch.float32 else _lib.BF16
+    _lib.check(lib.difflet_rocm_group_norm(xg.data_ptr(), torch.empty_like(xg).data_ptr(), dt, 2, pix,
+                                           c, groups, None, None, eps, 0, ws.data_ptr(), need,
+                                           torch.cuda.current_stream().cuda_stream), "group_norm")
+    stats = ws[-16 * groups:].view(torch.float32).cpu().double().view(2, 2, groups)
+    v = x.double().view(2, pix, groups, -1).transpose(1, 2).flatten(2)
+    ref = torch.stack([v.mean(-1), 1 / (v.var(-1, unbiased=False) + eps).sqrt()])
+    ulp = 2.0 ** (torch.frexp(ref).exponent.double() - 24)
+    assert ((stats - ref).abs() <= 0.51 * ulp).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
