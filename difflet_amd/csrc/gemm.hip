@@ -102,9 +102,9 @@ __host__ __device__ inline int sk_slot(const SkPlan& p, int c, int r, int gi) {
 constexpr int64_t SK_CTR_BYTES = 16384;        // one int counter per split tile
 constexpr int SK_MAX_TILES = (int)(SK_CTR_BYTES / 4);
 constexpr int64_t SK_SLOT_BYTES = 256 * 256 * 4;  // fp32 accumulators of one 256 x 256 tile
-constexpr int SK_MIN_STAGES = 6;               // shortest K range worth a workgroup
+constexpr int SK_MIN_STAGES = 8;               // shortest K range worth a workgroup (on average)
+constexpr int SK_MIN_STAGES_FEW = 6;            // the same with half of a group's workgroups idle
 constexpr int SK_MIN_SAVED_STAGES = 24;         // shortest cut off the busiest K walk (below)
-
 constexpr int SK_MIN_SAVED_OWN = 40;            // the same on scratch of the launch's own
 constexpr int SK_SAVED_ANYWAY = 48;             // a cut worth its partial sums in any launch
 constexpr int64_t SMALL_SCRATCH_CAP = 64LL << 20;  // fp32 sums of a small launch's K pieces
@@ -1028,20 +1028,27 @@ static int64_t sk_workspace_bytes(int groups) {
 // The schedule of T tiles of nk K stages (cut in units of `gran` stages) on `cus` compute
 // units. Whole tiles while the last wave of workgroups would still be >= 92 % full; otherwise
 // the full waves run whole tiles and the S tiles of the last one are cut over the XCDs (see
-// SkPlan), when each XCD's range is at least SK_MIN_STAGES stages and the cut takes a quarter
-// off the launch's K walk (waves * nu units on the busiest workgroup), and at least
+// SkPlan), when an XCD's range is at least SK_MIN_STAGES stages on average and the cut takes a
+// quarter off the launch's K walk (waves * nu units on the busiest workgroup), and at least
 // SK_MIN_SAVED_STAGES stages. The cut tiles' partial sums go through memory: 256 KB out and
 // back per cut, all CUs at once, which at ~6 TB/s costs about as much as 10-20 % of a
 // 3072-deep tile, whatever the K walk saves. On MI355X that pays on Qwen-Image's 336-tile
-// launches (FF2 MXFP8 365 -> 316 us, bf16 576 -> 483 us; 60 and 30 stages saved) and Wan's
-// 80-tile bf16 text k/v projection (93 -> 87 us, 40 saved), and loses on FLUX's 216-, 648-
-// and 864-tile ones (out projection bf16 87 -> 101 us, FF1 fp8 169 -> 198 us) and on the MXFP8
-// twin of that k/v projection (49 -> 66 us, 20 saved), which these rules leave whole. In a long
+// launches (FF2 MXFP8 365 -> 316 us, bf16 576 -> 483 us; 60 and 30 stages saved) and 80 bf16
+// tiles at K = 4096 (93 -> 87 us, 40 saved), and loses on FLUX's 216-, 648- and 864-tile ones
+// (out projection bf16 87 -> 101 us, FF1 fp8 169 -> 198 us) and on 80 MXFP8 tiles at K = 4096
+// (49 -> 66 us, 20 saved), which these rules leave whole. In a long
 // launch a quarter is more than it takes: SK_SAVED_ANYWAY stages saved pay whatever they are a part
 // of (5120 x 5120 over 14000 rows, 1100 tiles, 50 saved: 656 -> 606 us; at 42 saved, 3072 x 12288,
 // 1296 tiles ran 467 -> 461 and 1056 tiles 394 -> 402). A launch on scratch of its own (`own`) also
 // clears the counters and asks for SK_MIN_SAVED_OWN: 324 tiles at K = 3072, 30 saved, took 158 us
 // split and 151 whole; 264 tiles there, 42 saved, 150 whole and 131 split; at K = 12288 531 and 369.
+// Up to half a group of cut tiles writes so few partial sums that ranges of SK_MIN_STAGES_FEW pay
+// (whole -> cut at 48 stages, 1 to 16 tiles bf16 62 -> 44 to 66 -> 49 us, fp8 57 -> 46 to 63 -> 53,
+// MXFP8 62 -> 48 to 71 -> 58; 264 tiles bf16 145 -> 127); with more it comes out even at 20 to 24
+// and loses at 28 to 32 (30 tiles bf16 62 -> 66, fp8 60 -> 62; 288 tiles bf16 140 -> 153, fp8 131 ->
+// 148; 30 MXFP8 tiles of 32 stages 47 -> 59).
+static int sk_min_stages(int S, int g) { return 2 * S <= g ? SK_MIN_STAGES_FEW : SK_MIN_STAGES; }
+
 static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes, bool own = false) {
   const int nu = (nk + gran - 1) / gran;
   SkPlan pl = {T, 0, nu, gran, 0, 0, 0, 0};
@@ -1054,7 +1061,7 @@ static SkPlan sk_plan(int T, int nk, int gran, int cus, int64_t ws_bytes, bool o
   const int64_t units = (int64_t)ng * nu;
   const int64_t span = (units + NX - 1) / NX;
   if (S > SK_MAX_TILES || ws_bytes < sk_workspace_bytes(cus) ||
-      units / NX < std::max(1, SK_MIN_STAGES / gran) ||
+      units * gran < (int64_t)NX * std::max(gran, sk_min_stages(S, g)) ||
       (nu - span) * gran < (own ? SK_MIN_SAVED_OWN : SK_MIN_SAVED_STAGES) ||
       (4 * (nu - span) < (int64_t)waves * nu && (nu - span) * gran < SK_SAVED_ANYWAY))
     return pl;
@@ -1413,7 +1420,7 @@ extern "C" int difflet_rocm_gemm_schedule_check(int tiles, int k_stages, int gra
   for (int s = 0; s < pl.groups; ++s) {  // the kernel's walk
     const int c = s % pl.nx, r = s / pl.nx;
     const int64_t lo = sk_lo(pl, c), hi = sk_lo(pl, c + 1);
-    if (hi - lo < std::max(1, SK_MIN_STAGES / gran)) return 5;
+    if (hi - lo < 1 || (hi - lo + 1) * gran <= sk_min_stages(S, pl.g)) return 5;
     for (int64_t u = lo; u < hi;) {
       const int gi = (int)(u / pl.nu);
       const int64_t g0 = (int64_t)gi * pl.nu;

@@ -120,6 +120,16 @@ def test_gemm_split_plan_at_the_step_shapes():
         assert lib.difflet_rocm_gemm_schedule_check(336, nk, gran, 256, ws, ctypes.byref(dp),
                                                     ctypes.byref(groups)) == 0
         assert (dp.value, groups.value) == (336, 0)
+    # K ranges: 8 stages on average, 6 for up to half of the 32 tiles of a group (16 here, alone or
+    # behind a full wave); MXFP8's are stages too, not units of 4 rounded down
+    for tiles, nk, gran, cut in ((32, 64, 1, True), (32, 63, 1, False), (17, 63, 1, False),
+                                 (16, 48, 1, True), (16, 47, 1, False), (264, 48, 1, True),
+                                 (288, 48, 1, False), (32, 64, 4, True), (30, 32, 4, False),
+                                 (30, 60, 4, False), (16, 48, 4, True), (15, 44, 4, False),
+                                 (8, 32, 4, False)):
+        assert lib.difflet_rocm_gemm_schedule_check(tiles, nk, gran, 256, ws, ctypes.byref(dp),
+                                                    ctypes.byref(groups)) == 0
+        assert (groups.value > 0) is cut, (tiles, nk, gran)
     # without enough workspace nothing is split
     assert lib.difflet_rocm_gemm_schedule_check(336, 48, 1, 256, 1 << 20, ctypes.byref(dp),
                                                 ctypes.byref(groups)) == 0
