@@ -12,7 +12,7 @@ attention.py:8-48; the CUDA twin difflet/backends/cuda/ops_impl/attention.py:41-
 * Inputs ``(B, H, S, D)`` or ``(B*H, S, D)``, any strides with a contiguous last dim; softmax in
   fp32, output in ``v``'s dtype.
 
-The kernels run bf16 and fp16 on the matrix cores and fp32 on the vector ALUs (an fp32 model
+The kernels run bf16 and fp16 on the matrix cores and fp32 on the fp32 ones (an fp32 model
 computes in fp32, as the reference's CPU op does), at head_dim 128 (the DiTs) or 64 (the T5 /
 UMT5 text encoders). Any other head_dim up to 128 runs on the same kernels with q, k and v
 zero-padded to the next of those two: the padded dimensions add exact zeros to every score and

@@ -7,11 +7,11 @@ Same constructors, attributes, state dicts and bias semantics as the CPU twins
 ``reduce_dtype`` are accepted and have no effect at tp = 1.
 
 The matmul: bf16 weights run the bf16 kernels, one row of input (up to 8 at widths the GEMM would
-pad) through the GEMV kernel (the modulation and timestep linears, HBM-bound on W), more through
-the tiled GEMM; fp32
-weights (a model loaded in fp32, such as the T5 encoders' fp32 option) run the fp32
-matrix-core GEMM, in fp32 throughout as F.linear does. A K or N off the kernel's multiples (64
-and 4 for bf16, 4 and 4 for fp32) is zero-padded once on the weight (and per call on the input).
+pad, or laid out as it does not take them) through the GEMV kernel (the modulation and timestep
+linears, HBM-bound on W), more through the tiled GEMM; fp32 weights (a model loaded in fp32, such
+as the T5 encoders' fp32 option) run the fp32 matrix-core GEMM, in fp32 throughout as F.linear
+does. A K or N off the kernel's multiples (64 and 4 for bf16, 4 and 4 for fp32) is zero-padded once
+on the weight (and per call on the input).
 """
 
 from __future__ import annotations

@@ -9,8 +9,9 @@
 // two.
 //
 // A workgroup is 8 wavefronts over a BM x BN tile, in a 2 x 4 grid (4 x 2 for 256 rows: 64 x 64
-// each, the fewest LDS bytes per product) of MFMA tiles of 32 x 32 (operand roles and LDS swizzle as in gemm.hip: W first, A second, a
-// 128-byte K stage per row, chunk c of row r at c ^ swz8(r)). Stages go through a ring of NSLOT
+// each, the fewest LDS bytes per product) of MFMA tiles of 32 x 32 (operand roles and LDS swizzle
+// as in gemm.hip: W first, A second, a 128-byte K stage per row, chunk c of row r at c ^ swz8(r)).
+// Stages go through a ring of NSLOT
 // slots filled by direct-to-LDS loads, NSLOT - 1 of them in flight: these launches have one
 // workgroup per compute unit, so the ring alone has to cover the latency of cold weights.
 // One barrier per stage, before its last K step, whose fragments are in registers by then: each

@@ -394,11 +394,10 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
     workspace: None (every tile whole on one workgroup, the default), "call" (scratch of this
     call alone, from torch's allocator, where the launch gains by it, see _launch_scratch: safe on
     any stream and under graph capture), "shared" (the current stream's, see gemm_workspace) or
-    a zero-filled uint8 tensor of
-    difflet_rocm_gemm_workspace_bytes() bytes, which lets a launch whose last wave of tiles
-    would be poorly filled cut those tiles along K over the XCDs when that takes a quarter and
-    at least 24 K stages off its time (Qwen-Image's 336-tile projections, Wan's bf16 text k/v
-    projection; FLUX's launches stay whole)."""
+    a zero-filled uint8 tensor of difflet_rocm_gemm_workspace_bytes() bytes, which lets a launch
+    whose last wave of tiles would be poorly filled cut those tiles along K over the XCDs when that
+    takes a quarter and at least 24 K stages off its time, or 48 stages (Qwen-Image's 336-tile
+    projections; FLUX's launches stay whole). One problem of few tiles runs in smaller tiles."""
     # a problem without rows has nothing to compute (and an empty tensor may have no address)
     problems = [p for p in problems if p.a.shape[0] > 0]
     if not problems:
@@ -541,8 +540,7 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
            epilogue: int = _lib.EPI_NONE, gate: torch.Tensor | None = None,
            residual: torch.Tensor | None = None, act_col_start: int = 0,
-           rows_per_batch: int | None = None, out: torch.Tensor | None = None,
-           workspace: torch.Tensor | None | str = None) -> torch.Tensor:
+           rows_per_batch: int | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """bf16 ``x W^T + b`` over the last dim of x, with an optional fused epilogue."""
     x2 = _rows2d(x, "linear")
     n = w.shape[0]
@@ -550,7 +548,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
                                                 device=x.device)
     res2 = _rows2d(residual, "residual") if residual is not None else None
     gemm_grouped([Problem(x2, w, c, bias, gate, res2, rows_per_batch=rows_per_batch)],
-                 kind="bf16", epilogue=epilogue, act_col_start=act_col_start, workspace=workspace)
+                 kind="bf16", epilogue=epilogue, act_col_start=act_col_start)
     return c.reshape(*x.shape[:-1], n) if out is None else c
 
 

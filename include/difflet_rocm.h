@@ -61,12 +61,13 @@ int difflet_rocm_device_count(void);
  * (difflet/backends/cpu/ops_impl/attention.py:24-35). Masked scores take the dtype's lowest
  * finite value, so a fully masked row averages v exactly as the reference does.
  * workspace / workspace_bytes: optional device memory for the split schedule of attention,
- * unmasked or with bounds, over more than 1024 keys. When the launch's 256-query tiles would leave the last
- * wave of workgroups under 90 % full, one workgroup per compute unit runs the last round's
- * query tiles cut along the keys over lockstep sets of workgroups (the workgroups of a set read
+ * unmasked or with bounds, over more than 1024 keys. When the launch's 256-query tiles would leave
+ * the last wave of workgroups under 90 % full, one workgroup per compute unit runs the last
+ * round's query tiles cut along the keys over lockstep sets of workgroups (the workgroups of a set read
  * the same key tiles together), then the full rounds of whole tiles; query tiles cut
  * between sets are merged, in a fixed order, by the last contributor (a deterministic result;
- * the summation order differs from the unsplit one by fp32 rounding). With workspace NULL or too small every query tile runs whole.
+ * the summation order differs from the unsplit one by fp32 rounding). With workspace NULL or too
+ * small every query tile runs whole.
  * The workspace must be zero-filled once when allocated (the kernels leave it zeroed), and
  * launches that may overlap in time must not share one.
  * ---------------------------------------------------------------------------------------- */
@@ -222,14 +223,13 @@ typedef struct difflet_gemm_qk {
  * same K units of 32 neighbouring tiles together (whole-tile L2 sharing is kept). The cut is
  * made only when it takes a quarter and at least 24 K stages, or 48, off the launch's K walk
  * (Qwen-Image's 336-tile projections qualify; FLUX's 216-tile ones, which would save an
- * eighth, stay whole, and so does an MXFP8 projection of 512 rows at K = 4096). The workgroup
- * finishing a cut tile adds the fp32 partial sums of the others in a fixed order, so results
- * are deterministic for a given device. With workspace NULL (or too small) every tile runs
- * whole on one workgroup. A launch of one problem with few tiles (up to 4096 rows, epilogue NONE
- * or GATE_RESIDUAL, no fused q/k norm) runs in smaller tiles instead, and with a workspace may cut K into pieces, whose fp32 sums a second kernel
- * adds in order (nothing in the workspace need be zero for that, and its counters stay as they
- * are). The workspace must be zero-filled once when allocated; the GEMMs
- * leave it zeroed. Launches that may overlap in time (different streams) must not share one.
+ * eighth, stay whole). The workgroup finishing a cut tile adds the fp32 partial sums of the others
+ * in a fixed order, so results are deterministic for a given device. With workspace NULL (or too
+ * small) every tile runs whole on one workgroup. A launch of one problem with few tiles (up to 4096
+ * rows, epilogue NONE or GATE_RESIDUAL, no fused q/k norm) runs in smaller tiles instead, and with
+ * a workspace may cut K into pieces, whose fp32 sums a second kernel adds in order (nothing in the
+ * workspace need be zero for that, and its counters stay as they are). The workspace must be
+ * zero-filled once when allocated; the GEMMs leave it zeroed. Launches that may overlap in time (different streams) must not share one.
  * Returns the bytes needed on the current device: 16 KiB of counters + 2 x 256 KiB per compute
  * unit. No counterpart in the reference, whose linears call the vendor BLAS
  * (torch.nn.functional.linear, difflet/backends/cpu/ops_impl/linear.py:9-41). */
