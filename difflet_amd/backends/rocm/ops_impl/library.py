@@ -61,11 +61,12 @@ def _plain(*tensors: Optional[Tensor]) -> bool:
 _functorch_level = torch._C._functorch.peek_interpreter_stack
 _dispatch_modes = torch._C._len_torch_dispatch_stack
 _pre_dispatch_modes = torch._ops._len_torch_dispatch_stack_pre_dispatch
-_jit_trace = torch._C._get_tracing_state
+_jit_trace = torch._C._is_tracing
 _forward_ad = torch.autograd.forward_ad
-_below_autograd = torch._C._AutoDispatchBelowAutograd
-_SCALARS = frozenset((type(None), int, float, bool))
-_ARGUMENTS = _SCALARS | {Tensor, torch.nn.Parameter}
+_TENSORS = frozenset((Tensor, torch.nn.Parameter, type(None)))
+#: a twin is called at the device's key, below autograd as custom_op's implementations run: the
+#: kernel there is only for calls that come another way
+_DEVICE = torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
 
 
 def _eager() -> bool:
@@ -73,18 +74,14 @@ def _eager() -> bool:
     mode (make_fx, fake tensors), no functorch level (a batched tensor denies the gradient that
     the tensor under it needs), no forward-mode level."""
     return not (torch.compiler.is_compiling() or _functorch_level() is not None
-                or _dispatch_modes() or _pre_dispatch_modes() or _jit_trace() is not None
+                or _dispatch_modes() or _pre_dispatch_modes() or _jit_trace()
                 or _forward_ad._current_level >= 0)
 
 
-def _infer(op, twin, *args):
-    """twin(*args) where it can stand in for op, else op(*args). The twin runs below autograd, as
-    custom_op's implementations do: its kernel there is only for calls that come another way."""
-    if (_eager() and _ARGUMENTS.issuperset(map(type, args))  # no tensor subclass
-            and _plain(*[a for a in args if type(a) not in _SCALARS])):
-        with _below_autograd():
-            return twin(*args)
-    return op(*args)
+def _inference(*tensors: Optional[Tensor]) -> bool:
+    """Whether a twin can stand in for its custom_op: plain eager execution, plain device tensors
+    (no subclasses), no gradient."""
+    return _eager() and _TENSORS.issuperset(map(type, tensors)) and _plain(*tensors)
 
 
 # ---------------------------------------------------------------------------------- attention
@@ -108,8 +105,10 @@ _attention_infer = _infer_twin(_attention_op, _attention_impl, _attention_fake)
 def attention(q: Tensor, k: Tensor, v: Tensor, scale: float, causal: bool,
               attention_mask: Optional[Tensor], bound_min: Optional[Tensor],
               bound_max: Optional[Tensor]) -> Tensor:
-    return _infer(_attention_op, _attention_infer, q, k, v, scale, causal, attention_mask,
-                  bound_min, bound_max)
+    if _inference(q, k, v, attention_mask, bound_min, bound_max):
+        return _attention_infer.redispatch(_DEVICE, q, k, v, scale, causal, attention_mask,
+                                           bound_min, bound_max)
+    return _attention_op(q, k, v, scale, causal, attention_mask, bound_min, bound_max)
 
 
 def _attention_joint_impl(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
@@ -133,8 +132,10 @@ _attention_joint_infer = _infer_twin(_attention_joint_op, _attention_joint_impl,
 
 def attention_joint(q: Tensor, k: Tensor, v: Tensor, k2: Tensor, v2: Tensor, scale: float,
                     key_count: Optional[Tensor], count_offset: int) -> Tensor:
-    return _infer(_attention_joint_op, _attention_joint_infer, q, k, v, k2, v2, scale, key_count,
-                  count_offset)
+    if _inference(q, k, v, k2, v2, key_count):
+        return _attention_joint_infer.redispatch(_DEVICE, q, k, v, k2, v2, scale, key_count,
+                                                 count_offset)
+    return _attention_joint_op(q, k, v, k2, v2, scale, key_count, count_offset)
 
 
 # ------------------------------------------------------------------------------------- linear
@@ -155,19 +156,6 @@ def _gemv_fits(m: int, k: int, n: int) -> bool:
     return _gemv_stages(m, k) and (m == 1 or k % 64 != 0 or n % 4 != 0)
 
 
-def _gemm_reads(x: Tensor, w: Tensor, bias: Optional[Tensor]) -> bool:
-    """Whether the GEMM takes these operands: rows of x that do not overlap and start at multiples of
-    16 bytes (x with strided columns is copied first), a bias at a multiple of 8, operands below
-    4 GiB. The GEMV copies x, reads the bias value by value and takes a weight of any size."""
-    if x.dtype is not torch.bfloat16 or w.shape[0] * w.stride(0) >= 1 << 31:
-        return False
-    if x.stride(1) == 1 and not (x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
-                                 and x.shape[0] * x.stride(0) < 1 << 31 and x.data_ptr() % 16 == 0):
-        return False
-    return bias is None or (bias.dtype is torch.bfloat16 and bias.stride(0) == 1
-                            and bias.data_ptr() % 8 == 0)
-
-
 def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
     """y [M, out_features] bf16 = x [M, K'] @ w[:out_features, :K']^T + bias, where w [N', K'] may be
     the zero-padded weight (K' a multiple of 64, N' of 4); x is padded to K' here."""
@@ -175,9 +163,21 @@ def _linear_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int
     n_pad, k_pad = w.shape
     if m == 0:
         return x.new_empty((0, out_features), dtype=torch.bfloat16)
-    if n_pad == out_features and k_pad == kx and (
-            _gemv_fits(m, kx, n_pad) or (_gemv_stages(m, kx) and not _gemm_reads(x, w, bias))):
+    as_given = m <= GEMV_ROWS and n_pad == out_features and k_pad == kx
+    if as_given and _gemv_fits(m, kx, n_pad):
         return kernels.gemv(x, w, bias)
+    try:
+        return _linear_gemm(x, w, bias, out_features)
+    except (TypeError, ValueError, NotImplementedError):
+        # what the GEMM refuses (rows of x that overlap or are off 16 bytes, a bias off 8, 4 GiB and
+        # more) the GEMV takes: it copies x, reads the bias value by value, addresses in 64 bits
+        if as_given and _gemv_stages(m, kx):
+            return kernels.gemv(x, w, bias)
+        raise
+
+
+def _linear_gemm(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
+    kx, (n_pad, k_pad) = x.shape[1], w.shape
     if kx != k_pad:
         x = F.pad(x, (0, k_pad - kx))
     if bias is not None and bias.shape[0] != n_pad:
@@ -196,7 +196,9 @@ _linear_infer = _infer_twin(_linear_op, _linear_impl, _linear_fake)
 
 
 def linear(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
-    return _infer(_linear_op, _linear_infer, x, w, bias, out_features)
+    if _inference(x, w, bias):
+        return _linear_infer.redispatch(_DEVICE, x, w, bias, out_features)
+    return _linear_op(x, w, bias, out_features)
 
 
 def _linear_f32_impl(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
@@ -226,7 +228,9 @@ _linear_f32_infer = _infer_twin(_linear_f32_op, _linear_f32_impl, _linear_f32_fa
 
 
 def linear_f32(x: Tensor, w: Tensor, bias: Optional[Tensor], out_features: int) -> Tensor:
-    return _infer(_linear_f32_op, _linear_f32_infer, x, w, bias, out_features)
+    if _inference(x, w, bias):
+        return _linear_f32_infer.redispatch(_DEVICE, x, w, bias, out_features)
+    return _linear_f32_op(x, w, bias, out_features)
 
 
 def _fp8_linear_impl(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
@@ -252,7 +256,9 @@ _fp8_linear_infer = _infer_twin(_fp8_linear_op, _fp8_linear_impl, _fp8_linear_fa
 
 def fp8_linear(x: Tensor, w_kernel: Tensor, w_scale: Tensor, bias: Optional[Tensor],
                mx: bool) -> Tensor:
-    return _infer(_fp8_linear_op, _fp8_linear_infer, x, w_kernel, w_scale, bias, mx)
+    if _inference(x, w_kernel, w_scale, bias):
+        return _fp8_linear_infer.redispatch(_DEVICE, x, w_kernel, w_scale, bias, mx)
+    return _fp8_linear_op(x, w_kernel, w_scale, bias, mx)
 
 
 # ---------------------------------------------------------------------------- norms, rotary

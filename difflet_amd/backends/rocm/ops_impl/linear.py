@@ -79,7 +79,7 @@ class _RocmLinearBase(nn.Module):
             return x.new_empty(*shape[:-1], self.out_features)
         # a few rows run on the GEMV kernel with the weight as is; the GEMM reads the weight
         # zero-padded to its tile multiples (built once, only for odd shapes)
-        wg = w.detach() if library._gemv_fits(
+        wg = w.detach() if m <= library.GEMV_ROWS and library._gemv_fits(
             m, self.in_features, self.out_features) else self._weight_for_gemm()[0]
         y = library.linear(x2, wg, b, self.out_features)
         return y.reshape(*shape[:-1], self.out_features).to(x.dtype)

@@ -365,10 +365,13 @@ def _check_qk(qk: QkNormRope, problems: Sequence[Problem]) -> None:
             raise ValueError(f"problem {i}: RoPE rows [{lo}, {hi}) exceed the {rows}-row tables")
 
 
+_NEAR = 1 << 23  # a row stride up to which rows lie within 16 MB, whatever the element
+
+
 def _near_rows(t: torch.Tensor) -> torch.Tensor:
     """t, or a copy of it where its rows are over 16 MB apart (fewer than 256 rows, below the GEMMs'
     4 GiB: one token of each batch element, say), which the GEMM kernels do not address."""
-    if t.dim() == 2 and t.stride(0) * t.element_size() > 1 << 24 and t.shape[0] < 256:
+    if t.stride(0) * t.element_size() > 1 << 24 and t.shape[0] < 256:
         return t.contiguous()
     return t
 
@@ -439,12 +442,16 @@ def gemm_grouped(problems: Sequence[Problem], *, kind: str = "bf16",
         _check_qk(qk, problems)
     dev = _on_gpu(*[t for p in problems for t in (p.a, p.w, p.c, p.bias, p.gate, p.residual,
                                                   p.a_scale, p.w_scale)])
-    operands = [(_near_rows(p.a), _near_rows(p.w)) for p in problems]
+    copies = []  # of operands that the kernel does not address where they lie, until it is launched
     for i, p in enumerate(problems):
         q = arr[i]
-        a, w = operands[i]
-        q.a, q.lda = a.data_ptr(), a.stride(0)
-        q.w, q.ldw = w.data_ptr(), w.stride(0)
+        a, w, lda, ldw = p.a, p.w, p.a.stride(0), p.w.stride(0)
+        if lda > _NEAR or ldw > _NEAR:
+            a, w = _near_rows(a), _near_rows(w)
+            lda, ldw = a.stride(0), w.stride(0)
+            copies += [a, w]
+        q.a, q.lda = a.data_ptr(), lda
+        q.w, q.ldw = w.data_ptr(), ldw
         q.c, q.ldc = p.c.data_ptr(), p.c.stride(0)
         q.bias = p.bias.data_ptr() if p.bias is not None else None
         if p.gate is not None:
@@ -504,8 +511,8 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
     m, k = a.shape[0], w.shape[-1]
     n = w.shape[0]
     dev = a.device
-    a, w = _near_rows(a), _near_rows(w)
     y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    lda, ldw = a.stride(0), w.stride(0)
     kid = _KIND_ID[kind]
 
     def vec(t, dtype, length):
@@ -515,6 +522,7 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
     dts = _GEMM_A_DTYPES[kind]
     plain = (m > 0 and a.is_cuda and w.device == dev and a.dim() == 2 and w.dim() == 2
              and a.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1
+             and lda <= _NEAR and ldw <= _NEAR  # gemm_grouped copies others
              and a.dtype in dts and w.dtype in dts and (bias is None or vec(bias, torch.bfloat16, n)))
     if kid == 1:
         plain = (plain and a_scale is not None and w_scale is not None
@@ -530,7 +538,7 @@ def gemm_call(kind: str, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | 
         return y
     ws = _launch_scratch(kind, m, n, k, dev)
     check(lib().difflet_rocm_gemm_single(
-        kid, a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), n,
+        kid, a.data_ptr(), lda, w.data_ptr(), ldw, y.data_ptr(), n,
         None if bias is None else bias.data_ptr(), a_scale.data_ptr() if kid else None,
         w_scale.data_ptr() if kid else None, m, n, k, None if ws is None else ws.data_ptr(),
         0 if ws is None else ws.numel(), _raw_stream(dev)), f"gemm_{kind}")
